@@ -85,6 +85,7 @@ __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
     if (threadIdx.x < 64) {
         if (a.logits) {
             select_topk<1>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
+            __threadfence_block();  // lanes 0 .. topk - 1 wrote the choices
             if (lane == 0) {
                 const uint32_t y = blockIdx.y;
                 tile_meta[0] = sel_ids[y];

@@ -63,17 +63,6 @@ __device__ __forceinline__ float wave_max(float v) {
     auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
 }
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-    v = min(v, dpp_u32<0xB1>(v));
-    v = min(v, dpp_u32<0x4E>(v));
-    v = min(v, dpp_u32<0x124>(v));
-    v = min(v, dpp_u32<0x128>(v));
-    auto s16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = min((uint32_t)s16[0], (uint32_t)s16[1]);
-    auto s32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return min((uint32_t)s32[0], (uint32_t)s32[1]);
-}
-
 __device__ __forceinline__ bool finite_bits(float v) {
     return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
 }
@@ -82,58 +71,67 @@ __device__ __forceinline__ bool finite_bits(float v) {
 // generalised to k-of-E, E <= 256): repeatedly take the maximum, ties to the
 // lowest expert index; non-finite logits rank as -inf and turn every
 // probability NaN; chosen logits are rounded to bf16 and the probabilities
-// are bf16 of the softmax over the chosen k.  Lane 0 receives ids/probs.
+// are bf16 of the softmax over the chosen k.  Lane r holds the r-th choice
+// and writes its id and probability.
+//
+// Bound: one dependent chain per round (the wave-wide maximum).  The choices
+// stay one per lane and the lowest index of a maximum comes from a ballot: with
+// per-lane arrays indexed by the round the compiler kept them in scratch
+// memory, and a token's selection of 8 among 128 took about 11 us of a
+// 16-wavefront workgroup's time.
 template <int PER>  // logits per lane: experts <= 64 * PER
 __device__ void select_topk(const float *logits, uint32_t experts, uint32_t k, uint32_t *ids,
                             float *probs) {
     const uint32_t lane = threadIdx.x & 63;
     float v[PER];
-    bool avail[PER];
+    uint64_t avail[PER];  // experts not yet chosen (uniform)
     bool invalid = false;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        uint32_t e = lane + 64 * j;
-        float l = e < experts ? logits[e] : -INFINITY;
-        bool fin = finite_bits(l);
+        const uint32_t e = lane + 64 * j;
+        const float l = e < experts ? logits[e] : -INFINITY;
+        const bool fin = finite_bits(l);
         if (e < experts && !fin) invalid = true;
         v[j] = fin ? l : -INFINITY;
-        avail[j] = e < experts;
+        avail[j] = __ballot(e < experts);
     }
     invalid = __ballot(invalid) != 0;  // any lane saw a non-finite logit
-    float chosen[8];
-    uint32_t sel[8];
+    float chosen = 0.f;  // lane r: the r-th choice
+    uint32_t sel = 0;
     for (uint32_t r = 0; r < k; r++) {
         float m = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (avail[j]) m = fmaxf(m, v[j]);
-        m = wave_max(m);
-        uint32_t cand = 0xffffffffu;
+        for (int j = 0; j < PER; j++) m = fmaxf(m, v[j]);
+        m = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(m))));
+        // the lowest available expert with the maximum (a chosen one's value
+        // is -inf, which may be the maximum too, so availability counts)
+        uint32_t cand = 0;
+        bool found = false;
 #pragma unroll
-        for (int j = PER - 1; j >= 0; j--)
-            if (avail[j] && v[j] == m) cand = lane + 64 * j;
-        cand = wave_min_u32(cand);
-        sel[r] = cand;
-        chosen[r] = round_bf16(m);
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (lane + 64 * j == cand) avail[j] = false;
-    }
-    if (lane != 0) return;
-    for (uint32_t r = 0; r < k; r++)
-        if (!finite_bits(chosen[r])) invalid = true;
-    if (invalid) {
-        for (uint32_t r = 0; r < k; r++) {
-            ids[r] = sel[r] < experts ? sel[r] : 0;
-            probs[r] = __uint_as_float(0x7fc00000u);
+        for (int j = 0; j < PER; j++) {
+            const uint64_t at = __ballot(v[j] == m) & avail[j];
+            if (!found && at) {
+                const uint32_t b = (uint32_t)__builtin_ctzll(at);
+                cand = b + 64 * j;
+                found = true;
+                avail[j] &= ~(1ull << b);
+                if (lane == b) v[j] = -INFINITY;
+            }
         }
-        return;
+        if (lane == r) {
+            sel = cand;
+            chosen = round_bf16(m);
+        }
     }
+    if (__ballot(lane < k && !finite_bits(chosen))) invalid = true;
+    const float first = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(chosen)));
+    const float ex = expf(chosen - first);
     float sum = 0.f;
-    for (uint32_t r = 0; r < k; r++) sum += expf(chosen[r] - chosen[0]);
-    for (uint32_t r = 0; r < k; r++) {
-        ids[r] = sel[r];
-        probs[r] = round_bf16(expf(chosen[r] - chosen[0]) / sum);
+    for (uint32_t r = 0; r < k; r++)
+        sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ex), (int)r));
+    if (lane < k) {
+        ids[lane] = sel;
+        probs[lane] = invalid ? __uint_as_float(0x7fc00000u) : round_bf16(ex / sum);
     }
 }
 

@@ -1,0 +1,61 @@
+"""Routing kernels at the edges of their tiles, against the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from _util import Guarded, say
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(oco, a):
+    return oco.DeviceBuffer.from_array(np.ascontiguousarray(a))
+
+
+@pytest.mark.parametrize("experts,k", [(1, 1), (8, 8), (63, 8), (64, 8), (65, 8), (127, 5), (128, 8), (129, 8), (255, 7), (256, 8)])
+def test_route_select_lane_groups(lib, experts, k):
+    """Selections around the 64 experts that a lane group holds: random rows,
+    rows of few distinct values (ties within and across the groups go to the
+    lowest index), both zeros, and a row whose maximum sits in the last place."""
+    say("route_select lane groups", experts, k)
+    rng = np.random.default_rng(experts * 10 + k)
+    logits = rng.normal(size=(21, experts)).astype(np.float32)
+    logits[5:13] = rng.integers(-2, 2, (8, experts)).astype(np.float32)
+    logits[13] = np.where(np.arange(experts) % 2 == 0, -0.0, 0.0)
+    logits[14, -1] = 9.0
+    ids_b, probs_b = Guarded(lib, 21 * k * 4), Guarded(lib, 21 * k * 4)
+    lib.route_select(dev(lib, logits), 21, experts, k, ids_b.ptr, probs_b.ptr)
+    lib.synchronize()
+    want_ids, want_probs = O.select_experts(logits, k)
+    np.testing.assert_array_equal(ids_b.read(np.uint32).reshape(21, k), want_ids)
+    # probabilities are bf16: equal up to one bf16 step (exp is not bit-pinned)
+    np.testing.assert_allclose(probs_b.read(np.float32).reshape(21, k), want_probs, rtol=2 ** -7, atol=0)
+
+
+@pytest.mark.parametrize("fmt,tokens", [(12, 16), (12, 17), (12, 33), (39, 17)])
+def test_forward_selection_around_one_token_per_wavefront(lib, fmt, tokens):
+    """oco_experts_forward selects up to 16 tokens beside the route plan and
+    more in a launch of their own: both equal oco_router then
+    oco_experts_apply bit for bit."""
+    from oco_amd import synth
+    E, hidden, ffn, k = 128, 256, 256, 8
+    say("forward selection", fmt, tokens)
+    ws = [dev(lib, synth.weights(fmt, E * 256, 256, 40 + i)) for i in range(3)]
+    bank = lib.ExpertBank(fmt, hidden, ffn, E, k, *ws, activation=1, up_bias_one=False)
+    rng = np.random.default_rng(tokens)
+    x = dev(lib, O.f32_to_bf16(rng.normal(size=(tokens, hidden)).astype(np.float32)))
+    rw = dev(lib, (rng.normal(size=(E, hidden)) / 16).astype(np.float32))
+    rb = dev(lib, (rng.normal(size=E) * 0.1).astype(np.float32))
+    resid = O.f32_to_bf16(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    got = []
+    for whole in (True, False):
+        out, ids, probs = dev(lib, resid), lib.DeviceBuffer(tokens * k * 4), lib.DeviceBuffer(tokens * k * 4)
+        if whole:
+            bank.forward(rw, rb, x, lib.DType.BF16, tokens, out, ids, probs)
+        else:
+            lib.router(x, lib.DType.BF16, rw, rb, tokens, hidden, E, k, lib.DeviceBuffer(tokens * E * 4), ids, probs)
+            bank.apply(x, lib.DType.BF16, ids, probs, tokens, out)
+        lib.synchronize()
+        got.append((out.download(np.uint16), ids.download(np.uint32), probs.download(np.uint32)))
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
