@@ -116,6 +116,100 @@ __global__ __launch_bounds__(256) void router_logits_wide_kernel(const XT *x, co
     }
 }
 
+// The same logits on the matrix cores for prompts: bf16(x) and bf16(W) are
+// the operands as the reference rounds them, their products are exact in
+// f32, and each 32-column step's sum joins a 64-bit one, so that the result is
+// no further from the exact sum than the f32 chains' above (7.3e-8 relative
+// L2 at 2048 columns).  A workgroup takes 16 tokens x 16 experts; its
+// eight wavefronts take every eighth 32-column step, so that together they
+// read 256 consecutive columns of each row, and meet in LDS.  Rows past the
+// tokens or experts re-read the last one and are not stored.  Needs hidden %
+// 32 == 0 and 16-byte aligned rows.
+//
+// Bound by the latency of its loads (0.27 GFLOP over 3 MB for 512 x 128 x
+// 2048).  The kernel above re-reads each weight row per four tokens and pays
+// four FMAs per pair of values; it is the better one while tokens x experts
+// stays below about 8192 (both with the selection behind them, us: 32 x 128 x
+// 2048 7.6 above, 10.1 here; 128 x 32 x 2880 8.0, 12.5; 64 x 128 x 2048 about
+// 10, 10.2; 512 x 32 x 2880 about 18, 12.9; 512 x 128 x 2048 39, 10.9).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr uint64_t RM_MIN_LOGITS = 8192;
+constexpr int RM_TOKENS = 16, RM_EXPERTS = 16, RM_WAVES = 8, RM_DEPTH = 4;
+
+// Eight consecutive values of a row as loaded, and as a bf16 operand.
+template <typename XT>
+struct RouterRun;
+template <>
+struct RouterRun<float> {
+    float4 lo, hi;
+    __device__ __forceinline__ void load(const float *p) {
+        lo = *reinterpret_cast<const float4 *>(p);
+        hi = *reinterpret_cast<const float4 *>(p + 4);
+    }
+    __device__ __forceinline__ bf16x8 operand() const {
+        const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        uint16_t h[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) h[i] = f32_to_bf16_bits(f[i]);
+        bf16x8 v;
+        __builtin_memcpy(&v, h, 16);
+        return v;
+    }
+};
+template <>
+struct RouterRun<bf16_t> {
+    uint4 q;
+    __device__ __forceinline__ void load(const bf16_t *p) { q = *reinterpret_cast<const uint4 *>(p); }
+    __device__ __forceinline__ bf16x8 operand() const {
+        bf16x8 v;
+        __builtin_memcpy(&v, &q, 16);
+        return v;
+    }
+};
+
+template <typename XT>
+__global__ __launch_bounds__(64 * RM_WAVES) void router_logits_mfma_kernel(const XT *x, const float *w,
+                                                                           const float *bias, uint32_t tokens,
+                                                                           uint32_t hidden, uint32_t experts,
+                                                                           float *logits) {
+    __shared__ double part[RM_WAVES][RM_TOKENS][RM_EXPERTS + 1];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, c = (lane >> 4) * 8;
+    const uint32_t t0 = blockIdx.x * RM_TOKENS, e0 = blockIdx.y * RM_EXPERTS;
+    const XT *xr = x + (uint64_t)min(t0 + r, tokens - 1) * hidden + c;
+    const float *wr = w + (uint64_t)min(e0 + r, experts - 1) * hidden + c;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (uint32_t k0 = 32 * wave; k0 < hidden; k0 += 32 * RM_WAVES * RM_DEPTH) {
+        RouterRun<XT> a[RM_DEPTH];
+        RouterRun<float> b[RM_DEPTH];
+#pragma unroll
+        for (int u = 0; u < RM_DEPTH; u++) {  // every load of the round before its first product
+            const uint32_t k = min(k0 + 32 * RM_WAVES * u, hidden - 32);
+            a[u].load(xr + k);
+            b[u].load(wr + k);
+        }
+#pragma unroll
+        for (int u = 0; u < RM_DEPTH; u++)
+            if (k0 + 32 * RM_WAVES * u < hidden) {  // uniform
+                const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u].operand(), b[u].operand(),
+                                                                        f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] += (double)d[i];
+            }
+    }
+    // lane: expert r, tokens 4 (lane / 16) .. + 4
+#pragma unroll
+    for (int i = 0; i < 4; i++) part[wave][(lane >> 4) * 4 + i][r] = acc[i];
+    __syncthreads();
+    if (threadIdx.x >= RM_TOKENS * RM_EXPERTS) return;
+    const uint32_t t = threadIdx.x / RM_EXPERTS, e = threadIdx.x % RM_EXPERTS;
+    if (t0 + t >= tokens || e0 + e >= experts) return;
+    double v = 0.0;
+#pragma unroll
+    for (int q = 0; q < RM_WAVES; q++) v += part[q][t][e];
+    logits[(uint64_t)(t0 + t) * experts + e0 + e] = (float)v + (bias ? round_bf16(bias[e0 + e]) : 0.f);
+}
+
 // Route plan (routing.metal:4-39, nemotron.metal:238-273) by one workgroup:
 // per-expert route lists in route order, expert-sorted first rows, each
 // route's sorted row, (expert, first list row) tiles of `tile_rows`, and the
@@ -585,6 +679,16 @@ int router_logits_launch(const void *x, oco_dtype x_dtype, const float *w, const
     if (rec && hidden % 32) return fail(OCO_ERR_INVALID, "router: split rows need hidden %% 32 == 0 (hidden=%u)", hidden);
     const bool wide = hidden % 4 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & (xal - 1)) == 0 &&
                       (x_dtype == OCO_DT_F32 || x_dtype == OCO_DT_BF16);
+    if (logits && !rec && (uint64_t)tokens * experts >= RM_MIN_LOGITS && wide && hidden % 32 == 0 && ((uintptr_t)x & 15) == 0) {
+        const dim3 grid((tokens + RM_TOKENS - 1) / RM_TOKENS, (experts + RM_EXPERTS - 1) / RM_EXPERTS);
+        if (x_dtype == OCO_DT_F32)
+            hipLaunchKernelGGL(router_logits_mfma_kernel<float>, grid, dim3(64 * RM_WAVES), 0, s, (const float *)x, w,
+                               bias, tokens, hidden, experts, logits);
+        else
+            hipLaunchKernelGGL(router_logits_mfma_kernel<bf16_t>, grid, dim3(64 * RM_WAVES), 0, s, (const bf16_t *)x, w,
+                               bias, tokens, hidden, experts, logits);
+        return launch_check("router logits");
+    }
     if (wide || (rec && !logits)) {
         if (router_blocks + split_blocks >= 0x7fffffffull)
             return fail(OCO_ERR_INVALID, "router: %u tokens x %u experts over one grid", tokens, experts);

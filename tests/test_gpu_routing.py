@@ -59,3 +59,31 @@ def test_forward_selection_around_one_token_per_wavefront(lib, fmt, tokens):
         got.append((out.download(np.uint16), ids.download(np.uint32), probs.download(np.uint32)))
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("tokens,hidden,experts,dtype", [(64, 2048, 128, "bf16"), (257, 2880, 32, "f32"), (8192, 32, 1, "bf16"),
+                                                         (33, 1056, 255, "f32"), (500, 4096, 17, "bf16"), (37, 992, 256, "bf16")])
+def test_router_logits_of_a_prompt(lib, tokens, hidden, experts, dtype):
+    """tokens x experts past 8192: the matrix-core tiles at whole and partial
+    tiles of 16 x 16, with K steps that do and do not fill the eight
+    wavefronts.  Products of bf16 values are exact in f32; a 32-term sum in
+    f32 is within 32 u of the sum of magnitudes, and what follows is 64-bit
+    up to the result's own rounding."""
+    say("router prompt", tokens, hidden, experts, dtype)
+    rng = np.random.default_rng(hidden + experts)
+    x = rng.normal(size=(tokens, hidden)).astype(np.float32)
+    w = (rng.normal(size=(experts, hidden)) / np.sqrt(hidden)).astype(np.float32)
+    b = rng.normal(size=experts).astype(np.float32)
+    k = min(8, experts)
+    bits = O.f32_to_bf16(x)
+    logits = Guarded(lib, tokens * experts * 4)
+    ids, probs = lib.DeviceBuffer(tokens * k * 4), lib.DeviceBuffer(tokens * k * 4)
+    lib.router(dev(lib, bits if dtype == "bf16" else x), lib.DType.BF16 if dtype == "bf16" else lib.DType.F32, dev(lib, w),
+               dev(lib, b), tokens, hidden, experts, k, logits.ptr, ids, probs)
+    lib.synchronize()
+    got = logits.read(np.float32).reshape(tokens, experts)
+    as64 = lambda bits: (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)  # noqa: E731
+    xr, wr, br = as64(bits), as64(O.f32_to_bf16(w)), as64(O.f32_to_bf16(b))
+    want, mag = xr @ wr.T + br, np.abs(xr) @ np.abs(wr).T + np.abs(br)
+    assert np.all(np.abs(got - want) <= 34 * 2.0 ** -24 * mag)
+    np.testing.assert_array_equal(ids.download(np.uint32).reshape(tokens, k), O.select_experts(got, k)[0])
