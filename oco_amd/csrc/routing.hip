@@ -210,71 +210,187 @@ __global__ __launch_bounds__(64 * RM_WAVES) void router_logits_mfma_kernel(const
     logits[(uint64_t)(t0 + t) * experts + e0 + e] = (float)v + (bias ? round_bf16(bias[e0 + e]) : 0.f);
 }
 
-// Route plan (routing.metal:4-39, nemotron.metal:238-273) by one workgroup:
-// per-expert route lists in route order, expert-sorted first rows, each
+// ---- route plan (routing.metal:4-39, nemotron.metal:238-273) ---------------
+// Per-expert route lists in route order, expert-sorted first rows, each
 // route's sorted row, (expert, first list row) tiles of `tile_rows`, and the
-// two dispatch grids at words 0-5.  Routes are taken 1024 at a time; a
-// route's place in its expert's list is the expert's running count plus the
-// number of earlier routes of the chunk with the same expert, so lists keep
-// route order: up to 256 experts from ballot-matched peers inside each
-// wavefront and per-wavefront histograms in LDS, beyond that by broadcast
-// LDS reads of the whole chunk.  Ids >= experts are left out.
+// two dispatch grids at words 0-5.  Ids >= experts are left out.
 constexpr uint32_t PLAN_THREADS = 1024;
-constexpr uint32_t PLAN_HIST_EXPERTS = 256;  // per-wavefront histograms in LDS up to this many experts
-constexpr uint32_t PLAN_ONEPASS_CHUNKS = 8;   // the one-pass plan: up to this many chunks of 1024 routes
-constexpr uint32_t PLAN_ONEPASS_WORDS = 12288;  // and per-(chunk, wavefront, expert) counts up to this many words (48 KB)
+constexpr uint32_t PLAN_SPREAD_EXPERTS = 256, PLAN_SPREAD_CHUNKS = 64;  // the spread plan: experts, chunks of 1024 routes
+constexpr uint32_t PLAN_SELECT_TOKENS = PLAN_THREADS / 64;               // tokens selected beside the plan: one per wavefront
 
-__host__ __device__ inline bool plan_one_pass(uint32_t routes, uint32_t experts) {
-    const uint32_t nchunks = (routes + 1023) / 1024;
-    return experts <= PLAN_HIST_EXPERTS && nchunks <= PLAN_ONEPASS_CHUNKS && nchunks * 16 * experts <= PLAN_ONEPASS_WORDS;
+// The side job of the plan's launch: four elements (or one split item) and
+// one cleared word per thread t.
+__device__ __forceinline__ void plan_side_job(const PlanSide &side, uint64_t t) {
+    if (t < side.nzero) side.zero[t] = 0;
+    if (side.rec) {  // one split item (row, K step, block) per thread
+        if (t < (uint64_t)side.rows * ((side.k + 63) / 64) * 2) {
+            if (side.x_bf16)
+                mx6_split_item<uint16_t>(reinterpret_cast<const uint16_t *>(side.x), side.rec, side.k, t);
+            else
+                mx6_split_item<float>(reinterpret_cast<const float *>(side.x), side.rec, side.k, t);
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint64_t i = 4 * t + j;
+        if (i >= side.n) break;
+        const float v = side.x_bf16 ? __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(side.x)[i] << 16)
+                                    : reinterpret_cast<const float *>(side.x)[i];
+        const _Float16 h = (_Float16)v;
+        __builtin_memcpy(&side.y[i], &h, 2);
+    }
 }
+
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    v += dpp_u32<0xB1>(v);
+    v += dpp_u32<0x4E>(v);
+    v += dpp_u32<0x124>(v);
+    v += dpp_u32<0x128>(v);
+    auto s16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = (uint32_t)s16[0] + (uint32_t)s16[1];
+    auto s32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (uint32_t)s32[0] + (uint32_t)s32[1];
+}
+
+// The plan by one workgroup per expert (workgroups past the experts run the
+// side job): each counts all routes into an LDS histogram, sums the counts
+// and tiles of the experts before its own, and places its own expert's
+// routes: a route's place is the number of its expert's routes in earlier
+// (chunk of 1024, wavefront) slots plus those below its lane.  A decode
+// batch's selection (`side.logits`, at most PLAN_SELECT_TOKENS tokens) runs
+// in every workgroup, one token per wavefront; workgroup 0 stores it.
+//
+// Bound by its chain of loads, LDS passes and three barriers.  One workgroup
+// doing all experts' ballots, scan and scattered stores through one CU took
+// 11.8 us for 4,096 routes over 128 experts.
+__global__ __launch_bounds__(PLAN_THREADS) void route_plan_spread_kernel(const uint32_t *ids, uint32_t routes,
+                                                                         uint32_t experts, uint32_t tile_rows,
+                                                                         uint32_t up_tiles, uint32_t down_tiles,
+                                                                         uint32_t *plan, PlanSide side) {
+    if (blockIdx.x >= experts) {
+        plan_side_job(side, (uint64_t)(blockIdx.x - experts) * PLAN_THREADS + threadIdx.x);
+        return;
+    }
+    __shared__ uint32_t hist[PLAN_SPREAD_EXPERTS], slot[PLAN_SPREAD_CHUNKS * 16], before[2][4];
+    __shared__ uint32_t sel_id[PLAN_SELECT_TOKENS * 8];
+    __shared__ float sel_prob[PLAN_SELECT_TOKENS * 8];
+    const uint32_t own = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const uint32_t nchunks = (routes + PLAN_THREADS - 1) / PLAN_THREADS;
+    if (tid < PLAN_SPREAD_EXPERTS) hist[tid] = 0;
+    if (side.logits && wave < side.tokens) {
+        const float *lt = side.logits + (uint64_t)wave * experts;
+        uint32_t *it = sel_id + wave * side.topk;
+        float *pt = sel_prob + wave * side.topk;
+        if (experts <= 64)
+            select_topk<1>(lt, experts, side.topk, it, pt);
+        else if (experts <= 128)
+            select_topk<2>(lt, experts, side.topk, it, pt);
+        else
+            select_topk<4>(lt, experts, side.topk, it, pt);
+    }
+    __syncthreads();
+    if (side.logits && own == 0 && tid < routes) {
+        side.ids_out[tid] = sel_id[tid];
+        side.probs_out[tid] = sel_prob[tid];
+    }
+    auto expert_of = [&](uint32_t i) { return i >= routes ? 0xffffffffu : side.logits ? sel_id[i] : ids[i]; };
+
+    constexpr uint32_t KEEP = 4;  // chunks whose ids stay in registers for the placement
+    uint32_t ev[KEEP];
+#pragma unroll
+    for (uint32_t c = 0; c < KEEP; c++) ev[c] = expert_of(c * PLAN_THREADS + tid);
+    auto count = [&](uint32_t c, uint32_t e) {
+        const uint64_t mine = __ballot(e == own);
+        if (lane == 0) slot[c * 16 + wave] = (uint32_t)__popcll(mine);
+        if (e < experts) atomicAdd(&hist[e], 1u);
+    };
+#pragma unroll
+    for (uint32_t c = 0; c < KEEP; c++)
+        if (c < nchunks) count(c, ev[c]);  // uniform
+    for (uint32_t c = KEEP; c < nchunks; c++) count(c, expert_of(c * PLAN_THREADS + tid));
+    __syncthreads();
+    if (tid < PLAN_SPREAD_EXPERTS) {
+        const uint32_t n = hist[tid], tiles = n ? (n - 1) / tile_rows + 1 : 0;  // at most 65536 routes: 16 bits of tiles
+        const uint32_t rows = wave_sum_u32(tid < own ? n : 0u);
+        const uint32_t both = wave_sum_u32((tid < own ? tiles : 0u) | (tiles << 16));
+        if (lane == 0) {
+            before[0][wave] = rows;
+            before[1][wave] = both;
+        }
+    }
+    __syncthreads();
+    const uint32_t offs = before[0][0] + before[0][1] + before[0][2] + before[0][3];
+    const uint32_t both = before[1][0] + before[1][1] + before[1][2] + before[1][3];
+    const uint32_t tbase = both & 0xffffu, total = both >> 16, mine = hist[own];
+    const uint64_t grouped = 6 + 2 * ((uint64_t)(routes + 15) / 16 + experts);
+    const uint64_t list = grouped + (uint64_t)own * (routes + 1), sorted = grouped + (uint64_t)experts * (routes + 1);
+    const uint32_t DW = PLAN_DESC_HEAD + tile_rows;  // descriptor words per tile
+    if (tid == 0) {
+        plan[list] = mine;
+        plan[sorted + own] = offs;
+    }
+    for (uint32_t t = tid; (uint64_t)t * tile_rows < mine; t += PLAN_THREADS) {
+        const uint32_t b = t * tile_rows;
+        plan[6 + 2 * (uint64_t)(tbase + t)] = own;
+        plan[6 + 2 * (uint64_t)(tbase + t) + 1] = b;
+        if (side.desc) {
+            uint32_t *d = side.desc + (uint64_t)(tbase + t) * DW;
+            d[0] = own;
+            d[1] = min(tile_rows, mine - b);
+            d[2] = offs + b;
+            d[3] = b;
+        }
+    }
+    uint32_t placed = 0;  // this expert's routes in earlier chunks
+    auto place = [&](uint32_t c, uint32_t e) {
+        const uint64_t peers = __ballot(e == own);
+        const uint32_t v = lane < 16 ? slot[c * 16 + lane] : 0u;
+        const uint32_t s = wave_sum_u32((v << 16) | (lane < wave ? v : 0u));  // the chunk's, and earlier wavefronts'
+        if (e == own) {
+            const uint32_t i = c * PLAN_THREADS + tid;
+            const uint32_t pos = placed + (s & 0xffffu) + (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+            plan[list + 1 + pos] = i;
+            plan[sorted + experts + i] = offs + pos;
+            if (side.desc) side.desc[(uint64_t)(tbase + pos / tile_rows) * DW + PLAN_DESC_HEAD + pos % tile_rows] = i;
+        }
+        placed += s >> 16;
+    };
+#pragma unroll
+    for (uint32_t c = 0; c < KEEP; c++)
+        if (c < nchunks) place(c, ev[c]);  // uniform
+    for (uint32_t c = KEEP; c < nchunks; c++) place(c, expert_of(c * PLAN_THREADS + tid));
+    if (own == 0) {
+        if (tid == 0) {
+            plan[0] = up_tiles;
+            plan[1] = total;
+            plan[2] = 1;
+            plan[3] = down_tiles;
+            plan[4] = total;
+            plan[5] = 1;
+        }
+        if (side.desc) {  // unused tile slots: no rows
+            const uint32_t slots = (routes + 15) / 16 + experts;
+            for (uint32_t t = total + tid; t < slots; t += PLAN_THREADS) side.desc[(uint64_t)t * DW + 1] = 0;
+        }
+    }
+}
+
+// The plan by one workgroup, for more experts or routes than the spread plan
+// takes.  Routes are taken 1024 at a time; a route's place in its expert's
+// list is the expert's running count plus the number of earlier routes of
+// the chunk with the same expert: up to 256 experts from ballot-matched peers
+// inside each wavefront and per-wavefront histograms in LDS, beyond that by
+// broadcast LDS reads of the whole chunk.
+constexpr uint32_t PLAN_HIST_EXPERTS = 256;  // per-wavefront histograms in LDS up to this many experts
 
 __global__ __launch_bounds__(PLAN_THREADS) void route_plan_kernel(const uint32_t *ids, uint32_t routes,
                                                                   uint32_t experts, uint32_t tile_rows,
                                                                   uint32_t up_tiles, uint32_t down_tiles,
                                                                   uint32_t *plan, PlanSide side) {
-    if (blockIdx.x > 0) {  // the side job: four elements (or one split item) and one cleared word per thread
-        const uint64_t t = (uint64_t)(blockIdx.x - 1) * PLAN_THREADS + threadIdx.x;
-        if (t < side.nzero) side.zero[t] = 0;
-        if (side.rec) {  // one split item (row, K step, block) per thread
-            const uint64_t item = t;
-            if (item < (uint64_t)side.rows * ((side.k + 63) / 64) * 2) {
-                if (side.x_bf16)
-                    mx6_split_item<uint16_t>(reinterpret_cast<const uint16_t *>(side.x), side.rec, side.k, item);
-                else
-                    mx6_split_item<float>(reinterpret_cast<const float *>(side.x), side.rec, side.k, item);
-            }
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint64_t i = 4 * t + j;
-            if (i >= side.n) break;
-            const float v = side.x_bf16 ? __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(side.x)[i] << 16)
-                                        : reinterpret_cast<const float *>(side.x)[i];
-            const _Float16 h = (_Float16)v;
-            __builtin_memcpy(&side.y[i], &h, 2);
-        }
+    if (blockIdx.x > 0) {
+        plan_side_job(side, (uint64_t)(blockIdx.x - 1) * PLAN_THREADS + threadIdx.x);
         return;
-    }
-    // The expert selection first, a token per wavefront; the plan then reads
-    // the selected ids back (written and read by this workgroup only).
-    if (side.logits) {
-        const uint32_t wave0 = threadIdx.x >> 6;
-        for (uint32_t t = wave0; t < side.tokens; t += PLAN_THREADS / 64) {
-            const float *lt = side.logits + (uint64_t)t * experts;
-            uint32_t *it = side.ids_out + (uint64_t)t * side.topk;
-            float *pt = side.probs_out + (uint64_t)t * side.topk;
-            if (experts <= 64)
-                select_topk<1>(lt, experts, side.topk, it, pt);
-            else if (experts <= 128)
-                select_topk<2>(lt, experts, side.topk, it, pt);
-            else
-                select_topk<4>(lt, experts, side.topk, it, pt);
-        }
-        __threadfence_block();
-        __syncthreads();
-        ids = side.ids_out;
     }
     // LDS: chunk ids [1024]; run, tile base, offset [experts]; per-wavefront
     // histograms [16][experts] (experts <= PLAN_HIST_EXPERTS)
@@ -285,75 +401,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_kernel(const uint32_t
     const uint64_t grouped = 6 + 2 * ((uint64_t)(routes + 15) / 16 + experts);
     const uint64_t sorted = grouped + (uint64_t)experts * (routes + 1);
 
-    // One pass (experts <= PLAN_HIST_EXPERTS, up to PLAN_ONEPASS_CHUNKS chunks
-    // of 1024 routes whose per-wavefront histograms fit the LDS): every
-    // route's rank among its wavefront's peers by ballots, the counts per
-    // (chunk, wavefront, expert) in LDS, one exclusive scan per expert over
-    // those slots (which also gives the counts), then every placement at
-    // once -- a handful of barriers instead of four per chunk.
-    const uint32_t nchunks = (routes + PLAN_THREADS - 1) / PLAN_THREADS;
-    const bool one_pass = plan_one_pass(routes, experts);
-    uint32_t ev[PLAN_ONEPASS_CHUNKS], rk[PLAN_ONEPASS_CHUNKS];
-    if (one_pass) {
-        // counts of (chunk, wavefront) slot q of expert e at hist[e * HS + q]:
-        // an odd row stride keeps the scan's reads (threads of several
-        // experts, each over a run of slots) on distinct banks
-        const uint32_t slots = nchunks * 16, HS = slots + 1;
-        for (uint32_t t = tid; t < HS * experts; t += PLAN_THREADS) hist[t] = 0;
-        const uint32_t id_bits = experts > 1 ? 32u - (uint32_t)__builtin_clz(experts - 1) : 0u;
-#pragma unroll
-        for (uint32_t c = 0; c < PLAN_ONEPASS_CHUNKS; c++) {
-            ev[c] = 0xffffffffu;
-            rk[c] = 0;
-            if (c < nchunks) {
-                const uint32_t i = c * PLAN_THREADS + tid;
-                ev[c] = i < routes ? ids[i] : 0xffffffffu;
-            }
-        }
-        __syncthreads();  // hist cleared
-#pragma unroll
-        for (uint32_t c = 0; c < PLAN_ONEPASS_CHUNKS; c++) {
-            if (c >= nchunks) break;  // uniform
-            const uint32_t e = ev[c];
-            uint64_t peers = __ballot(e < experts);
-            if (e >= experts) peers = ~peers;
-            for (uint32_t bit = 0; bit < id_bits; bit++) {
-                const uint64_t b = __ballot((e >> bit) & 1u);
-                peers &= ((e >> bit) & 1u) ? b : ~b;
-            }
-            rk[c] = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
-            if (e < experts && (peers >> lane) == 1ull) hist[e * HS + c * 16 + wave] = rk[c] + 1;
-        }
-        __syncthreads();
-        // exclusive scan per expert over the slots (chunk, wavefront) in
-        // route order: G consecutive threads per expert, each over a run of
-        // slots, joined by a shuffle scan within the group
-        uint32_t G = 1;
-        while (G * 2 * experts <= PLAN_THREADS && G < 64) G *= 2;
-        const uint32_t e = tid / G, j = tid % G, per = (slots + G - 1) / G;
-        uint32_t local = 0;
-        if (e < experts)
-            for (uint32_t q = j * per; q < min(slots, j * per + per); q++) local += hist[e * HS + q];
-        uint32_t incl = local;
-        for (uint32_t o = 1; o < G; o <<= 1) {
-            const uint32_t v = (uint32_t)__shfl_up((int)incl, o, (int)G);
-            if (j >= o) incl += v;
-        }
-        if (e < experts) {
-            uint32_t run_e = incl - local;
-            for (uint32_t q = j * per; q < min(slots, j * per + per); q++) {
-                const uint32_t v = hist[e * HS + q];
-                hist[e * HS + q] = run_e;
-                run_e += v;
-            }
-            if (j == G - 1) run[e] = incl;
-        }
-        __syncthreads();
-    }
     // 1. counts per expert (four ids in flight per thread)
-    for (uint32_t e = tid; e < experts && !one_pass; e += PLAN_THREADS) run[e] = 0;
+    for (uint32_t e = tid; e < experts; e += PLAN_THREADS) run[e] = 0;
     __syncthreads();
-    for (uint32_t base = tid; base < routes && !one_pass; base += 4 * PLAN_THREADS) {
+    for (uint32_t base = tid; base < routes; base += 4 * PLAN_THREADS) {
         uint32_t ev[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -430,36 +481,6 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_kernel(const uint32_t
         uint32_t total = 0;  // tiles in use: the per-wavefront tile sums of step 2
         for (uint32_t w = 0; w < 16; w++) total += wsum[16 + w];
         for (uint32_t t = total + tid; t < slots; t += PLAN_THREADS) side.desc[(uint64_t)t * DW + 1] = 0;
-    }
-    if (one_pass) {
-        __syncthreads();  // offs[] is complete
-        // Every route's place goes to an expert-sorted array in LDS first,
-        // (expert << 16) | route, and the lists and descriptors are written
-        // from it in sorted order: consecutive threads then store consecutive
-        // words, where storing from each route's own thread scatters every
-        // wavefront instruction over 64 lines through this one CU's address
-        // unit.
-        uint32_t *srt = hist + max(16 * experts, (nchunks * 16 + 1) * experts);
-#pragma unroll
-        for (uint32_t c = 0; c < PLAN_ONEPASS_CHUNKS; c++) {
-            if (c >= nchunks) break;  // uniform
-            const uint32_t e = ev[c], i = c * PLAN_THREADS + tid;
-            if (e < experts) {
-                const uint32_t pos = hist[e * (nchunks * 16 + 1) + c * 16 + wave] + rk[c];
-                srt[offs[e] + pos] = (e << 16) | i;
-                plan[sorted + experts + i] = offs[e] + pos;
-            }
-        }
-        uint32_t placed = 0;  // routes with a valid expert: the per-wavefront count sums of step 2
-        for (uint32_t w = 0; w < 16; w++) placed += wsum[w];
-        __syncthreads();
-        for (uint32_t j = tid; j < placed; j += PLAN_THREADS) {
-            const uint32_t v = srt[j], e = v >> 16, i = v & 0xffffu, pos = j - offs[e];
-            plan[grouped + (uint64_t)e * (routes + 1) + 1 + pos] = i;
-            if (side.desc)
-                side.desc[(uint64_t)(tbase[e] + pos / tile_rows) * DW + PLAN_DESC_HEAD + pos % tile_rows] = i;
-        }
-        return;
     }
     __syncthreads();
     for (uint32_t e = tid; e < experts; e += PLAN_THREADS) run[e] = 0;  // reused as the running count of step 3
@@ -607,10 +628,11 @@ int route_plan_launch(const uint32_t *ids, uint32_t routes, uint32_t experts, ui
                     "oco_route_plan: need 0 < experts <= 4096 and tile_rows >= 16 (the plan holds ceil(routes/16) + "
                     "experts tiles)");
     PlanSide sj = side ? *side : PlanSide{};
-    // The plan's workgroup selects at most one token per wavefront (a decode
-    // batch, which saves the launch).  More tokens are spread over the chip:
-    // 512 tokens of 8 among 128 took 350 us as 32 rounds of that workgroup.
-    if (sj.logits && sj.tokens > PLAN_THREADS / 64) {
+    const bool spread = experts <= PLAN_SPREAD_EXPERTS && routes <= PLAN_SPREAD_CHUNKS * PLAN_THREADS;
+    // The spread plan selects at most one token per wavefront (a decode
+    // batch, which saves the launch).  More tokens take a launch of their own:
+    // 512 tokens of 8 among 128 took 350 us as 32 rounds of one workgroup.
+    if (sj.logits && (!spread || sj.tokens > PLAN_SELECT_TOKENS)) {
         OCO_TRY(route_select_launch(sj.logits, sj.tokens, experts, sj.topk, sj.ids_out, sj.probs_out, stream));
         sj.logits = nullptr;
         ids = sj.ids_out;
@@ -619,14 +641,14 @@ int route_plan_launch(const uint32_t *ids, uint32_t routes, uint32_t experts, ui
     const uint64_t side_items = sj.rec ? (uint64_t)sj.rows * ((sj.k + 63) / 64) * 2 : (sj.n + 3) / 4;  // threads
     const uint64_t side_blocks =
         std::max<uint64_t>((side_items + PLAN_THREADS - 1) / PLAN_THREADS, (sj.nzero + PLAN_THREADS - 1) / PLAN_THREADS);
-    if (side_blocks >= 0x7fffffffu) return fail(OCO_ERR_INVALID, "oco_route_plan: side job of %llu elements", (unsigned long long)sj.n);
-    // LDS words: chunk ids, run / tile base / offset per expert, then the
-    // histograms and (one pass) the expert-sorted routes.
-    const size_t lds = (size_t)(PLAN_THREADS + 3 * experts +
-                                (plan_one_pass(routes, experts)
-                                     ? std::max(16 * experts, ((routes + 1023) / 1024 * 16 + 1) * experts) + routes
-                                 : experts <= PLAN_HIST_EXPERTS ? 16 * experts
-                                                                : 0)) * 4;
+    if (side_blocks >= 0x7fffffffu - experts) return fail(OCO_ERR_INVALID, "oco_route_plan: side job of %llu elements", (unsigned long long)sj.n);
+    if (spread) {
+        hipLaunchKernelGGL(route_plan_spread_kernel, dim3(experts + (unsigned)side_blocks), dim3(PLAN_THREADS), 0, stream,
+                           ids, routes, experts, tile_rows, up_tiles, down_tiles, plan, sj);
+        return launch_check("oco_route_plan");
+    }
+    // LDS words: chunk ids, run / tile base / offset per expert, histograms
+    const size_t lds = (size_t)(PLAN_THREADS + 3 * experts + (experts <= PLAN_HIST_EXPERTS ? 16 * experts : 0)) * 4;
     if (lds > 64 * 1024)
         OCO_TRY(hip_check(hipFuncSetAttribute((const void *)route_plan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                           "hipFuncSetAttribute"));

@@ -87,3 +87,32 @@ def test_router_logits_of_a_prompt(lib, tokens, hidden, experts, dtype):
     want, mag = xr @ wr.T + br, np.abs(xr) @ np.abs(wr).T + np.abs(br)
     assert np.all(np.abs(got - want) <= 34 * 2.0 ** -24 * mag)
     np.testing.assert_array_equal(ids.download(np.uint32).reshape(tokens, k), O.select_experts(got, k)[0])
+
+
+@pytest.mark.parametrize("routes,experts,tile", [(1, 1, 16), (64, 256, 16), (1025, 3, 48), (4096, 128, 32), (5000, 200, 64),
+                                                 (65536, 256, 16), (65537, 256, 16), (300, 257, 32), (70, 7, 1 << 31)])
+def test_route_plan_spread_and_single_workgroup(lib, routes, experts, tile):
+    """The plan by one workgroup per expert (up to 256 experts and 65536
+    routes) and past both limits by one workgroup, some ids >= experts."""
+    say("route_plan edges", routes, experts, tile)
+    rng = np.random.default_rng(routes)
+    ids = rng.integers(0, experts, routes).astype(np.uint32)
+    ids[rng.random(routes) < 0.03] = experts + 5
+    words = lib.route_plan_words(routes, experts)
+    out = Guarded(lib, words * 4)
+    lib.route_plan(dev(lib, ids), routes, experts, tile, 3, 4, out.ptr)
+    lib.synchronize()
+    got = out.read(np.uint32)
+    grouped = 6 + 2 * ((routes + 15) // 16 + experts)
+    rows = grouped + experts * (routes + 1)
+    tiles, offset = [], 0
+    for e in range(experts):
+        mine = np.nonzero(ids == e)[0]
+        base = grouped + e * (routes + 1)
+        assert got[base] == mine.size and got[rows + e] == offset
+        np.testing.assert_array_equal(got[base + 1:base + 1 + mine.size], mine)
+        np.testing.assert_array_equal(got[rows + experts + mine], offset + np.arange(mine.size))
+        tiles += [(e, b) for b in range(0, mine.size, tile)]
+        offset += mine.size
+    np.testing.assert_array_equal(got[:6], [3, len(tiles), 1, 4, len(tiles), 1])
+    np.testing.assert_array_equal(got[6:6 + 2 * len(tiles)].reshape(-1, 2), np.array(tiles, np.uint32).reshape(-1, 2))
