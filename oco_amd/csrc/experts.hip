@@ -30,7 +30,7 @@ struct MoeArgs {
     const uint8_t *w[2];     // gated: {gate, up}; otherwise {down, unused}
     const float *logits;     // single token: select the experts in-kernel
     const uint32_t *ids;     // [routes] expert per route (no plan, no logits)
-    const uint32_t *plan;    // route plan (tile = (expert, first row)) or null (tile = route)
+    const uint32_t *desc;    // the route plan's tile descriptors (tiles of up to T routes) or null (tile = route)
     uint32_t k, n, experts, topk;
     const void *x;           // activations
     uint32_t x_bf16;         // activation element type
@@ -59,8 +59,6 @@ __device__ __forceinline__ float activation(uint32_t act, float g, float u) {
     float sig = (g < 0 ? e : 1.0f) / (1.0f + e);
     return sig * g * u;
 }
-
-constexpr uint32_t PLAN_TILE = 16;  // routes per route-plan tile (its minimum, see oco_route_plan)
 
 template <int FMT, bool GATED, int T, int NPL>
 __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
@@ -97,25 +95,11 @@ __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
                         a.probs_out[r] = sel_probs[r];
                     }
             }
-        } else if (a.plan) {
-            if (lane == 0) {
-                // Plan tiles hold up to PLAN_TILE routes; each is served as
-                // PLAN_TILE / T sub-tiles of T routes.
-                const uint32_t y = blockIdx.y / (PLAN_TILE / T), sub = blockIdx.y % (PLAN_TILE / T);
-                const uint32_t ntiles = a.plan[1];
-                uint32_t count = 0, expert = 0;
-                if (y < ntiles) {
-                    expert = a.plan[6 + 2 * y];
-                    const uint32_t first = a.plan[7 + 2 * y] + sub * T;
-                    const uint64_t grouped = 6 + 2 * ((uint64_t)(a.routes + 15) / 16 + a.experts);
-                    const uint64_t base = grouped + (uint64_t)expert * (a.routes + 1);
-                    const uint32_t total = a.plan[base];
-                    count = first < total ? min((uint32_t)T, total - first) : 0u;
-                    for (uint32_t j = 0; j < count; j++) tile_routes[j] = a.plan[base + 1 + first + j];
-                }
-                tile_meta[0] = expert;
-                tile_meta[1] = count;
-            }
+        } else if (a.desc) {
+            // one read: {expert, rows, first sorted row, first list row, route ids}
+            const uint32_t v = lane < PLAN_DESC_HEAD + T ? a.desc[(uint64_t)blockIdx.y * (PLAN_DESC_HEAD + T) + lane] : 0u;
+            if (lane < 2) tile_meta[lane] = v;
+            if (lane >= PLAN_DESC_HEAD && lane < PLAN_DESC_HEAD + T) tile_routes[lane - PLAN_DESC_HEAD] = v;
         } else if (lane == 0) {
             tile_meta[0] = a.ids[blockIdx.y];
             tile_meta[1] = 1;
@@ -356,7 +340,7 @@ static int moe_launch(uint32_t fmt, bool gated, MoeArgs a, uint32_t tiles, uint3
     const int npl = (int)((pieces + 31) / 32);
     // Without a plan every tile is one route: a one-route kernel, whose
     // staged activations take a quarter of the LDS.
-    const int t = a.plan ? MOE_T : 1;
+    const int t = a.desc ? MOE_T : 1;
     MoeFn fn = npl <= 4 ? moe_pick_format(fmt, gated, npl, t) : nullptr;
     if (!fn)
         return fail(OCO_ERR_UNSUPPORTED, "experts: format %u with k=%u has no routed kernel (rows over %u bytes)",
@@ -452,6 +436,8 @@ uint64_t oco_experts_workspace(const oco_experts *w, uint32_t tokens) {
     uint64_t bytes = align256(oco_route_plan_words((uint32_t)routes, w->experts) * 4) + align256(routes * w->ffn * 4) +
                      align256((uint64_t)tokens * w->hidden * 2) + align256(routes * 4) + align256(routes * w->hidden * 4);
     if (w->format == OCO_Q4_K) bytes += align256(routes * w->ffn * 2);
+    if (w->format != OCO_MXFP4)  // the routed kernel's tile descriptors
+        bytes += align256(plan_desc_words((uint32_t)routes, w->experts, MOE_T) * 4);
     if (w->format == OCO_MXFP4)  // ... and the plan's tile descriptors (tiles of up to 32 rows)
         bytes += align256(mx_rows_bytes(tokens, w->hidden)) + align256(mx_rows_bytes((uint32_t)routes, w->ffn)) +
                  align256(plan_desc_words((uint32_t)routes, w->experts, 32) * 4);
@@ -662,7 +648,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
     }
 
     uint32_t tiles = routes, parallel = routes;
-    const uint32_t *use_plan = nullptr;
+    const uint32_t *tile_desc = nullptr;
     if (fused_select) {
         // expert_expand (projections.metal:78-137): every gate/up workgroup
         // selects the token's experts from the logits; workgroup (0, 0)
@@ -705,9 +691,17 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
         return oco_moe_sum(down, OCO_DT_F32, probs, out, w->hidden, tokens, w->k, stream);
     }
     if (tokens > 1) {
-        OCO_TRY(route_plan_launch(ids, routes, w->experts, PLAN_TILE, 0, 0, plan, &sel, s));
-        use_plan = plan;
-        tiles = ((routes + PLAN_TILE - 1) / PLAN_TILE + w->experts) * (PLAN_TILE / MOE_T);
+        // Tiles of MOE_T routes from descriptors, one workgroup row per slot
+        // of their bound.  (The plan's own 16-route tiles, each as four
+        // sub-tiles over ceil(routes / 16) + experts slots, made 520 rows of
+        // workgroups for the 32 routes of a 4-token batch over 128 experts,
+        // nearly all of which read the plan and left: gate/up 42.9 us, down 37.)
+        uint32_t *desc = (uint32_t *)(xrec + (w->format == OCO_Q4_K ? align256((uint64_t)routes * w->ffn * 2) : 0));
+        PlanSide side = sel;
+        side.desc = desc;
+        OCO_TRY(route_plan_launch(ids, routes, w->experts, MOE_T, 0, 0, plan, &side, s));
+        tile_desc = desc;
+        tiles = (uint32_t)plan_desc_slots(routes, w->experts, MOE_T);
         parallel = std::min(routes, w->experts);
     }
     MoeArgs a = {};
@@ -721,7 +715,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
     a.out0 = act;
     a.out1 = nullptr;
     a.ids = ids;
-    a.plan = use_plan;
+    a.desc = tile_desc;
     a.k = w->hidden;
     a.n = w->ffn;
     a.experts = w->experts;

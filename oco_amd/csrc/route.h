@@ -16,8 +16,9 @@ namespace oco {
 // and per-tile descriptors (`desc` set), so that a tile's consumer finds all
 // it needs in one contiguous read: PLAN_DESC_HEAD words {expert, rows (0 for
 // an unused tile slot), first sorted row, first list row} then the tile's
-// `tile_rows` route ids in list order, for every one of the plan's
-// ceil(routes / 16) + experts tile slots.
+// `tile_rows` route ids in list order, for each of plan_desc_slots tile
+// slots.  With descriptors the plan's own (expert, first row) pairs are not
+// written, and tiles may hold fewer than 16 rows.
 struct PlanSide {
     const void *x;
     uint32_t x_bf16;
@@ -34,8 +35,16 @@ struct PlanSide {
     uint32_t *desc;
 };
 constexpr uint32_t PLAN_DESC_HEAD = 4;
+// Descriptor slots: the plan's tile slots, or for tiles of fewer than 16
+// rows the bound sum over experts of ceil(count / tile_rows).
+__host__ __device__ inline uint64_t plan_desc_slots(uint32_t routes, uint32_t experts, uint32_t tile_rows) {
+    if (tile_rows >= 16) return (uint64_t)(routes + 15) / 16 + experts;
+    const uint64_t hit = routes < experts ? routes : experts;
+    const uint64_t bound = (routes + (uint64_t)(tile_rows - 1) * hit) / tile_rows;
+    return bound < routes ? bound : routes;
+}
 __host__ __device__ inline uint64_t plan_desc_words(uint32_t routes, uint32_t experts, uint32_t tile_rows) {
-    return ((uint64_t)(routes + 15) / 16 + experts) * (PLAN_DESC_HEAD + tile_rows);
+    return plan_desc_slots(routes, experts, tile_rows) * (PLAN_DESC_HEAD + tile_rows);
 }
 
 // Router logits [tokens, experts] (routing.metal:96-146) into `logits` (or

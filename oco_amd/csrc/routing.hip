@@ -272,7 +272,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_spread_kernel(const u
         plan_side_job(side, (uint64_t)(blockIdx.x - experts) * PLAN_THREADS + threadIdx.x);
         return;
     }
-    __shared__ uint32_t hist[PLAN_SPREAD_EXPERTS], slot[PLAN_SPREAD_CHUNKS * 16], before[2][4];
+    __shared__ uint32_t hist[PLAN_SPREAD_EXPERTS], slot[PLAN_SPREAD_CHUNKS * 16], before[3][4];
     __shared__ uint32_t sel_id[PLAN_SELECT_TOKENS * 8];
     __shared__ float sel_prob[PLAN_SELECT_TOKENS * 8];
     const uint32_t own = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -311,18 +311,19 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_spread_kernel(const u
     for (uint32_t c = KEEP; c < nchunks; c++) count(c, expert_of(c * PLAN_THREADS + tid));
     __syncthreads();
     if (tid < PLAN_SPREAD_EXPERTS) {
-        const uint32_t n = hist[tid], tiles = n ? (n - 1) / tile_rows + 1 : 0;  // at most 65536 routes: 16 bits of tiles
+        const uint32_t n = hist[tid], tiles = n ? (n - 1) / tile_rows + 1 : 0;  // at most 65536 routes
         const uint32_t rows = wave_sum_u32(tid < own ? n : 0u);
-        const uint32_t both = wave_sum_u32((tid < own ? tiles : 0u) | (tiles << 16));
+        const uint32_t pairs = wave_sum_u32(tid < own ? tiles : 0u), all = wave_sum_u32(tiles);
         if (lane == 0) {
             before[0][wave] = rows;
-            before[1][wave] = both;
+            before[1][wave] = pairs;
+            before[2][wave] = all;
         }
     }
     __syncthreads();
     const uint32_t offs = before[0][0] + before[0][1] + before[0][2] + before[0][3];
-    const uint32_t both = before[1][0] + before[1][1] + before[1][2] + before[1][3];
-    const uint32_t tbase = both & 0xffffu, total = both >> 16, mine = hist[own];
+    const uint32_t tbase = before[1][0] + before[1][1] + before[1][2] + before[1][3];
+    const uint32_t total = before[2][0] + before[2][1] + before[2][2] + before[2][3], mine = hist[own];
     const uint64_t grouped = 6 + 2 * ((uint64_t)(routes + 15) / 16 + experts);
     const uint64_t list = grouped + (uint64_t)own * (routes + 1), sorted = grouped + (uint64_t)experts * (routes + 1);
     const uint32_t DW = PLAN_DESC_HEAD + tile_rows;  // descriptor words per tile
@@ -332,9 +333,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_spread_kernel(const u
     }
     for (uint32_t t = tid; (uint64_t)t * tile_rows < mine; t += PLAN_THREADS) {
         const uint32_t b = t * tile_rows;
-        plan[6 + 2 * (uint64_t)(tbase + t)] = own;
-        plan[6 + 2 * (uint64_t)(tbase + t) + 1] = b;
-        if (side.desc) {
+        if (!side.desc) {
+            plan[6 + 2 * (uint64_t)(tbase + t)] = own;
+            plan[6 + 2 * (uint64_t)(tbase + t) + 1] = b;
+        } else {
             uint32_t *d = side.desc + (uint64_t)(tbase + t) * DW;
             d[0] = own;
             d[1] = min(tile_rows, mine - b);
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_spread_kernel(const u
             plan[5] = 1;
         }
         if (side.desc) {  // unused tile slots: no rows
-            const uint32_t slots = (routes + 15) / 16 + experts;
+            const uint32_t slots = (uint32_t)plan_desc_slots(routes, experts, tile_rows);
             for (uint32_t t = total + tid; t < slots; t += PLAN_THREADS) side.desc[(uint64_t)t * DW + 1] = 0;
         }
     }
@@ -465,9 +467,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_kernel(const uint32_t
     for (uint32_t e = tid; e < experts; e += PLAN_THREADS) {
         uint32_t t = tbase[e];
         for (uint32_t b = 0; b < run[e]; b += tile_rows, t++) {
-            plan[6 + 2 * (uint64_t)t] = e;
-            plan[6 + 2 * (uint64_t)t + 1] = b;
-            if (side.desc) {
+            if (!side.desc) {
+                plan[6 + 2 * (uint64_t)t] = e;
+                plan[6 + 2 * (uint64_t)t + 1] = b;
+            } else {
                 uint32_t *d = side.desc + (uint64_t)t * DW;
                 d[0] = e;
                 d[1] = min(tile_rows, run[e] - b);
@@ -477,7 +480,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void route_plan_kernel(const uint32_t
         }
     }
     if (side.desc) {  // unused tile slots: no rows
-        const uint32_t slots = (routes + 15) / 16 + experts;
+        const uint32_t slots = (uint32_t)plan_desc_slots(routes, experts, tile_rows);
         uint32_t total = 0;  // tiles in use: the per-wavefront tile sums of step 2
         for (uint32_t w = 0; w < 16; w++) total += wsum[16 + w];
         for (uint32_t t = total + tid; t < slots; t += PLAN_THREADS) side.desc[(uint64_t)t * DW + 1] = 0;
@@ -623,7 +626,7 @@ static int route_select_launch(const float *logits, uint32_t tokens, uint32_t ex
 int route_plan_launch(const uint32_t *ids, uint32_t routes, uint32_t experts, uint32_t tile_rows, uint32_t up_tiles,
                       uint32_t down_tiles, uint32_t *plan, const PlanSide *side, hipStream_t stream) {
     if (!ids || !plan) return fail(OCO_ERR_INVALID, "oco_route_plan: null pointer");
-    if (experts == 0 || experts > 4096 || tile_rows < 16)
+    if (experts == 0 || experts > 4096 || tile_rows == 0 || (tile_rows < 16 && !(side && side->desc)))
         return fail(OCO_ERR_INVALID,
                     "oco_route_plan: need 0 < experts <= 4096 and tile_rows >= 16 (the plan holds ceil(routes/16) + "
                     "experts tiles)");
