@@ -82,7 +82,10 @@ __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
     // Which expert and which routes this workgroup serves.
     if (threadIdx.x < 64) {
         if (a.logits) {
-            select_topk<1>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
+            if (a.experts <= 64)
+                select_topk<1>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
+            else
+                select_topk<4>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
             __threadfence_block();  // lanes 0 .. topk - 1 wrote the choices
             if (lane == 0) {
                 const uint32_t y = blockIdx.y;
@@ -481,12 +484,9 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
         return fail(OCO_ERR_INVALID, "%s: workspace of %llu bytes, need %llu", who,
                     (unsigned long long)workspace_bytes, (unsigned long long)oco_experts_workspace(w, tokens));
     oco_stream stream = (oco_stream)s;
-    // Selection inside the gate/up kernel covers one token over <= 64 experts;
-    // otherwise it runs in the route plan's workgroup, before the plan.
     const bool small = mx_small_path(w, tokens);
-    const bool fused_select = logits && tokens == 1 && w->experts <= 64 && !small;
-    PlanSide sel = {};
-    if (logits && !fused_select) {
+    PlanSide sel = {};  // the selection beside the route plan
+    if (logits) {
         sel.logits = logits;
         sel.tokens = tokens;
         sel.topk = w->k;
@@ -649,7 +649,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
 
     uint32_t tiles = routes, parallel = routes;
     const uint32_t *tile_desc = nullptr;
-    if (fused_select) {
+    if (logits && tokens == 1) {
         // expert_expand (projections.metal:78-137): every gate/up workgroup
         // selects the token's experts from the logits; workgroup (0, 0)
         // records ids and probabilities for the down pass and the combine.

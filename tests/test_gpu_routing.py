@@ -116,3 +116,33 @@ def test_route_plan_spread_and_single_workgroup(lib, routes, experts, tile):
         offset += mine.size
     np.testing.assert_array_equal(got[:6], [3, len(tiles), 1, 4, len(tiles), 1])
     np.testing.assert_array_equal(got[6:6 + 2 * len(tiles)].reshape(-1, 2), np.array(tiles, np.uint32).reshape(-1, 2))
+
+
+@pytest.mark.parametrize("fmt,E", [(12, 65), (12, 128), (12, 256), (39, 128), (8, 64)])
+def test_forward_one_token_over_many_experts(lib, fmt, E):
+    """One token selects inside the gate/up kernel whatever the number of
+    experts: ids, probabilities and rows equal oco_router then
+    oco_experts_apply bit for bit."""
+    from oco_amd import synth
+    hidden, ffn, k = 256, 256, 8
+    say("forward one token", fmt, E)
+    ws = [dev(lib, synth.weights(fmt, E * 256, 256, 60 + i)) for i in range(3)]
+    bank = lib.ExpertBank(fmt, hidden, ffn, E, k, *ws, activation=1, up_bias_one=False)
+    rng = np.random.default_rng(E)
+    x = dev(lib, O.f32_to_bf16(rng.normal(size=(1, hidden)).astype(np.float32)))
+    rw = dev(lib, (rng.normal(size=(E, hidden)) / 16).astype(np.float32))
+    rb = dev(lib, np.where(np.arange(E) == E - 1, 9.0, 0.0).astype(np.float32))  # the last expert is chosen first
+    resid = O.f32_to_bf16(rng.normal(size=(1, hidden)).astype(np.float32))
+    got = []
+    for whole in (True, False):
+        out, ids, probs = dev(lib, resid), dev(lib, np.zeros(k, np.uint32)), lib.DeviceBuffer(k * 4)
+        if whole:
+            bank.forward(rw, rb, x, lib.DType.BF16, 1, out, ids, probs)
+        else:
+            lib.router(x, lib.DType.BF16, rw, rb, 1, hidden, E, k, lib.DeviceBuffer(E * 4), ids, probs)
+            bank.apply(x, lib.DType.BF16, ids, probs, 1, out)
+        lib.synchronize()
+        got.append((out.download(np.uint16), ids.download(np.uint32), probs.download(np.uint32)))
+    assert got[0][1][0] == E - 1
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
