@@ -21,6 +21,7 @@
 
 #include "formats.h"
 #include "matmul.h"
+#include "skinny.h"
 
 namespace oco {
 
@@ -769,14 +770,19 @@ static void operand_launch(const void *w, uint64_t row_bytes, uint32_t n, uint32
                        n, k, wo, (const uint16_t *)x, xo, xchunks, wblocks);
 }
 
+static int vendor_workspace_check(const void *workspace, uint64_t bytes, uint64_t need) {
+    if (!workspace || bytes < need)
+        return fail(OCO_ERR_INVALID, "oco_matmul_ws: workspace of %llu bytes, need %llu", (unsigned long long)bytes,
+                    (unsigned long long)need);
+    return OCO_OK;
+}
+
 static int vendor_matmul(uint32_t format, const void *w, const void *x, oco_dtype x_dtype, void *y, oco_dtype y_dtype,
                          const float *bias, const oco_matrix *p, const BlasPlan &pl, void *workspace,
                          uint64_t workspace_bytes, hipStream_t stream) {
     const uint32_t m = p->m, n = p->n, k = p->k;
     const VendorLayout v = vendor_layout(format, x_dtype, m, n, k, pl.ws);
-    if (!workspace || workspace_bytes < v.total)
-        return fail(OCO_ERR_INVALID, "oco_matmul_ws: workspace of %llu bytes, need %llu",
-                    (unsigned long long)workspace_bytes, (unsigned long long)v.total);
+    OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));
     uint8_t *ws = (uint8_t *)workspace;
     const bool gain = q4_gain(format, n, x_dtype);
     uint16_t *wo = format == OCO_F16 ? nullptr : (uint16_t *)(ws + v.w);
@@ -902,6 +908,15 @@ static const BlasPlan *vendor_plan(uint32_t format, oco_dtype x_dtype, const oco
     return pl.ok ? &pl : nullptr;
 }
 
+// Fewer rows than the dequantize pass pays for go to the few-row kernel,
+// unless an override asks for one of the two paths below it.  (Against the
+// fused tiles, bf16 out, us: Q4_K 12288 x 4096 at 8 rows 52 -> 14.7.)
+static bool use_skinny(uint32_t format, const oco_matrix *p) {
+    int32_t ov[4];
+    return p->m < 32 && !plan_override(OCO_KNOB_MATMUL_VENDOR, ov) && !plan_override(OCO_KNOB_MATMUL_TILE, ov) &&
+           skinny_fits(format, p->m, p->n, p->k);
+}
+
 extern "C" uint64_t oco_matmul_workspace(uint32_t format, oco_dtype x_dtype, const oco_matrix *p) {
     if (!p || as_matvec(format, x_dtype, p)) return 0;
     if (use_mx(format)) return mx_workspace_bytes(p->m, p->n, p->k);
@@ -927,7 +942,23 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     // 16-byte aligned for it; otherwise the fused tiles run.
     const bool aligned = (format != OCO_F16 || ((uintptr_t)w & 15) == 0) &&
                          (x_dtype != OCO_DT_F16 || ((uintptr_t)x & 15) == 0);
-    if (const BlasPlan *pl = aligned ? vendor_plan(format, x_dtype, p) : nullptr)
+    const BlasPlan *pl = aligned ? vendor_plan(format, x_dtype, p) : nullptr;
+    if (use_skinny(format, p)) {
+        const void *xin = x;
+        float *inv = nullptr;
+        if (pl && q4_gain(format, p->n, x_dtype)) {  // scaled f16 rows through the workspace, as the vendor path makes them
+            const VendorLayout v = vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws);
+            OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));
+            uint16_t *xo = (uint16_t *)((uint8_t *)workspace + v.x);
+            inv = (float *)((uint8_t *)workspace + v.gain);
+            hipLaunchKernelGGL(row_gain_f16_kernel, dim3(p->m), dim3(256), 0, (hipStream_t)stream, (const uint16_t *)x, xo, inv, p->k);
+            OCO_TRY(launch_check("oco_matmul: row gains"));
+            xin = xo;
+        }
+        return skinny_launch(format, w, xin, x_dtype == OCO_DT_F16 || inv, y, y_dtype == OCO_DT_BF16, p->has_bias ? bias : nullptr,
+                             inv, p->m, p->n, p->k, (hipStream_t)stream);
+    }
+    if (pl)
         return vendor_matmul(format, w, x, x_dtype, y, y_dtype, bias, p, *pl, workspace, workspace_bytes,
                              (hipStream_t)stream);
     return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
@@ -939,7 +970,7 @@ extern "C" int oco_matmul(uint32_t format, const void *w, const void *x, oco_dty
     if (p->m == 0 || p->n == 0) return OCO_OK;
     if (as_matvec(format, x_dtype, p)) return oco_matvec(format, w, x, x_dtype, y, y_dtype, bias, nullptr, p, stream);
     const uint64_t need = oco_matmul_workspace(format, x_dtype, p);
-    if (!need) return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
+    if (!need) return oco_matmul_ws(format, w, x, x_dtype, y, y_dtype, bias, p, nullptr, 0, stream);
     void *ws = nullptr;
     OCO_TRY(hip_check(hipMallocAsync(&ws, need, (hipStream_t)stream), "oco_matmul: hipMallocAsync"));
     const int rc = oco_matmul_ws(format, w, x, x_dtype, y, y_dtype, bias, p, ws, need, stream);
