@@ -21,6 +21,7 @@
 
 #include "formats.h"
 #include "matmul.h"
+#include "panel.h"
 #include "skinny.h"
 
 namespace oco {
@@ -637,16 +638,17 @@ __global__ __launch_bounds__(256) void row_gain_f16_kernel(const uint16_t *x, ui
     for (uint32_t i = threadIdx.x; i < k; i += 256) orow[i] = operand_bits<false>(bf16_bits_to_f32(xr[i]) * gain);
 }
 
-// y[m, n] = acc (* 1 / row gain) + bf16(bias), as f32 or bf16: four columns
-// per thread.
-__global__ __launch_bounds__(256) void gemm_epilogue_kernel(const float *acc, const float *bias, const float *inv_gain,
-                                                            void *y, bool y_bf16, uint32_t n, uint64_t quads) {
+// y[m, n] = sum of the `parts` f32 products at acc (* 1 / row gain) +
+// bf16(bias), as f32 or bf16: four columns per thread.
+__global__ __launch_bounds__(256) void gemm_epilogue_kernel(const float *acc, uint32_t parts, const float *bias,
+                                                            const float *inv_gain, void *y, bool y_bf16, uint32_t n,
+                                                            uint64_t quads) {
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= quads) return;
     const uint32_t col = (uint32_t)(4 * i % n);
     const float g = inv_gain ? inv_gain[4 * i / n] : 1.0f;
-    const float4 v = *reinterpret_cast<const float4 *>(acc + 4 * i);
-    float r[4] = {v.x, v.y, v.z, v.w};
+    f32x4 r = *reinterpret_cast<const f32x4 *>(acc + 4 * i);
+    for (uint32_t p = 1; p < parts; p++) r += *reinterpret_cast<const f32x4 *>(acc + 4 * (i + p * quads));
 #pragma unroll
     for (int j = 0; j < 4; j++) r[j] = r[j] * g + (bias ? round_bf16(bias[col + j]) : 0.f);
     if (y_bf16)
@@ -813,9 +815,37 @@ static int vendor_matmul(uint32_t format, const void *w, const void *x, oco_dtyp
     if (st != HIPBLAS_STATUS_SUCCESS) return fail(OCO_ERR_HIP, "oco_matmul: hipblasLtMatmul status %d", (int)st);
     if (!direct) {
         const uint64_t quads = (uint64_t)m * n / 4;
-        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, acc,
+        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, acc, 1u,
                            p->has_bias ? bias : nullptr, inv, y, y_dtype == OCO_DT_BF16, n, quads);
         OCO_TRY(launch_check("oco_matmul: epilogue"));
+    }
+    return OCO_OK;
+}
+
+// The panel kernel in place of the dequantize pass, the GEMM and the
+// epilogue: the same workspace, of which it takes the f16 activations and
+// (K parts) the f16 weights' place.
+static int panel_matmul(uint32_t format, const PanelPlan &pp, const void *w, const void *x, oco_dtype x_dtype, void *y,
+                        oco_dtype y_dtype, const float *bias, const oco_matrix *p, const VendorLayout &v, void *workspace,
+                        hipStream_t stream) {
+    const uint32_t m = p->m, n = p->n, k = p->k;
+    uint8_t *ws = (uint8_t *)workspace;
+    const bool gain = q4_gain(format, n, x_dtype);
+    uint16_t *xo = (uint16_t *)(ws + v.x);
+    float *inv = gain ? (float *)(ws + v.gain) : nullptr, *part = (float *)(ws + v.w);
+    const float *b = p->has_bias ? bias : nullptr;
+    if (gain)
+        hipLaunchKernelGGL(row_gain_f16_kernel, dim3(m), dim3(256), 0, stream, (const uint16_t *)x, xo, inv, k);
+    else if (x_dtype == OCO_DT_BF16)
+        operand_launch<OCO_F16>(nullptr, 0, n, k, nullptr, x, xo, (uint64_t)m * k / 8, stream);
+    OCO_TRY(launch_check("oco_matmul: f16 activations"));
+    const uint16_t *xin = gain || x_dtype == OCO_DT_BF16 ? xo : (const uint16_t *)x;
+    OCO_TRY(panel_launch(format, pp, w, xin, y, y_dtype == OCO_DT_BF16, b, inv, part, m, n, k, stream));
+    if (pp.splits > 1) {
+        const uint64_t quads = (uint64_t)m * n / 4;
+        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, part,
+                           pp.splits, b, inv, y, y_dtype == OCO_DT_BF16, n, quads);
+        OCO_TRY(launch_check("oco_matmul: sum of the parts"));
     }
     return OCO_OK;
 }
@@ -917,6 +947,12 @@ static bool use_skinny(uint32_t format, const oco_matrix *p) {
            skinny_fits(format, p->m, p->n, p->k);
 }
 
+static PanelPlan use_panel(uint32_t format, const oco_matrix *p) {
+    int32_t ov[4];
+    if (plan_override(OCO_KNOB_MATMUL_VENDOR, ov) || plan_override(OCO_KNOB_MATMUL_TILE, ov)) return {};
+    return panel_plan(format, p->m, p->n, p->k);
+}
+
 extern "C" uint64_t oco_matmul_workspace(uint32_t format, oco_dtype x_dtype, const oco_matrix *p) {
     if (!p || as_matvec(format, x_dtype, p)) return 0;
     if (use_mx(format)) return mx_workspace_bytes(p->m, p->n, p->k);
@@ -957,6 +993,14 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
         }
         return skinny_launch(format, w, xin, x_dtype == OCO_DT_F16 || inv, y, y_dtype == OCO_DT_BF16, p->has_bias ? bias : nullptr,
                              inv, p->m, p->n, p->k, (hipStream_t)stream);
+    }
+    if (pl) {
+        const PanelPlan pp = use_panel(format, p);
+        if (pp.mt) {
+            const VendorLayout v = vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws);
+            OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));
+            return panel_matmul(format, pp, w, x, x_dtype, y, y_dtype, bias, p, v, workspace, (hipStream_t)stream);
+        }
     }
     if (pl)
         return vendor_matmul(format, w, x, x_dtype, y, y_dtype, bias, p, *pl, workspace, workspace_bytes,

@@ -1,0 +1,263 @@
+// Y[m, n] = X[m, k] W[n, k]^T for a prompt chunk, weights decoded on the way
+// into the matrix cores: the f16 operands of the dequantize pass (half(w),
+// half(x)) and fp32 accumulation, without the pass's n x k x 2 bytes of f16
+// weights to memory and back, and with the bias and the output type in the
+// kernel.  Replaces the large tiles of DenseMatrix::apply
+// (src/weights/compute/matrix.rs:130-379).
+//
+// A workgroup of four wavefronts, one per SIMD, covers 16 MT activation rows
+// x 64 NT weight rows.  The wavefronts split the weight rows, so each weight
+// is decoded once per workgroup, in the registers of the lane whose MFMA
+// fragment it fills (units.h); the activations are shared: 256 columns of
+// them per step go straight to LDS (global_load_lds), two steps of them, each
+// row's 16-byte runs rotated by XOR with the row so that 16 rows read
+// conflict-free.  One barrier per 256 columns; the next step's weights and
+// activations are requested during a step's products.
+// Bound by the SIMD's issue: per 32 columns and wavefront 16 MT NT clocks of
+// MFMA and about 80 NT of decode (Q4_K), which do not overlap on one SIMD.
+#include "panel.h"
+
+#include <cmath>
+
+#include "units.h"
+
+namespace oco {
+
+struct PanelArgs {
+    const uint8_t *w;
+    const uint16_t *x;  // f16 rows
+    uint32_t n, k, m, row_bytes;
+    uint32_t mtiles, splits;  // row tiles; K parts
+    void *y;
+    const float *bias;
+    const float *inv;   // per-row factor of the result or null
+    float *part;        // K parts: f32 [splits][m][n] (y, bias and inv unused)
+    uint32_t y_bf16;
+};
+
+// s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima
+__device__ __forceinline__ void panel_vm_wait() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
+
+template <int B, int E, typename F>
+__device__ __forceinline__ void panel_for(F &&f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        panel_for<B + 1, E>(f);
+    }
+}
+
+template <int FMT, int MT, int NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void panel_kernel(KPRE_PARAMS, PanelArgs a) {
+    KPRE_APPLY(a);
+    using U = WeightUnit<FMT>;
+    constexpr int BM = 16 * MT, XL = BM / 8;  // 16-byte activation loads per lane and step
+    // Separate arrays, so that the compiler can tell reads of one step's
+    // activations from the asynchronous loads into the other.
+    __shared__ __attribute__((aligned(16))) uint8_t xs0[BM * 512], xs1[BM * 512];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    // workgroups that share weights (the row tiles of a column tile) run on one XCD
+    const uint32_t lin = xcd_order(blockIdx.x, gridDim.x);
+    const uint32_t mt = lin % a.mtiles, rest = lin / a.mtiles, part = rest % a.splits, ct = rest / a.splits;
+    const uint32_t m0 = mt * BM, n0 = ct * 64 * NT, rows = min(a.n - n0, 64u * NT);
+    const uint32_t all = a.k / 256, u0 = (uint32_t)((uint64_t)part * all / a.splits),
+                   u1 = (uint32_t)((uint64_t)(part + 1) * all / a.splits);
+    RowSrc ws;
+    ws.r = uniform_rsrc(a.w + (uint64_t)n0 * a.row_bytes, rows * a.row_bytes);
+    uint32_t wrow[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) wrow[t] = min((wave * NT + t) * 16 + r, rows - 1) * a.row_bytes;
+    // activation load i of a step: LDS rows 2 (wave + 4 i), + 1; slot s of row
+    // R holds run s ^ (R % 16)
+    gbytes xsrc[XL];
+#pragma unroll
+    for (int i = 0; i < XL; i++) {
+        const uint32_t R = 2 * (wave + 4 * i) + (lane >> 5), run = (lane & 31) ^ (R & 15);
+        xsrc[i] = gp(reinterpret_cast<const uint8_t *>(a.x)) + (uint64_t)min(m0 + R, a.m - 1) * a.k * 2 + 16 * run;
+    }
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // The requests for step u: NT weight units, then XL activation loads.
+    // Past the last step the weights read nothing and the activations repeat it.
+    auto item = [&](auto kk, uint32_t u, uint8_t *xs, U *w) __attribute__((always_inline)) {
+        constexpr int K = decltype(kk)::value;
+        if constexpr (K < NT) {
+            w[K].load(ws, u < u1 ? wrow[K] + u * U::UNIT : UNIT_OFF, q, 256);
+        } else {
+            constexpr int i = K - NT;
+            __builtin_amdgcn_global_load_lds((const GLOBAL void *)(xsrc[i] + (uint64_t)min(u, u1 - 1) * 512),
+                                             (__attribute__((address_space(3))) void *)(xs + (wave + 4 * i) * 1024), 16, 0, 0);
+        }
+    };
+    constexpr int ITEMS = NT + XL, RUNS = 6;  // spread over the first six of a step's eight runs
+    auto step = [&](uint32_t u, const uint8_t *xs, U *w, uint8_t *xn, U *wn) __attribute__((always_inline)) {
+        panel_vm_wait();                          // this step's activations are in LDS, its weights here
+        asm volatile("s_barrier" ::: "memory");  // ... in every wavefront; the other buffer is free
+#pragma unroll
+        for (int t = 0; t < NT; t++) w[t].prep(q);
+        panel_for<0, 8>([&](auto cc) __attribute__((always_inline)) {
+            constexpr int C = decltype(cc)::value;
+            if constexpr (C < RUNS)
+                panel_for<C * ITEMS / RUNS, (C + 1) * ITEMS / RUNS>([&](auto kk) { item(kk, u + 1, xn, wn); });
+            f16x8 xv[MT];
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                xv[i] = *reinterpret_cast<const f16x8 *>(xs + (16 * i + r) * 512 + 16 * ((U::col(q, C) / 8) ^ r));
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                uint32_t o[4];
+                w[t].run(C, o);
+                f16x8 wv;
+                __builtin_memcpy(&wv, o, 16);
+#pragma unroll
+                for (int i = 0; i < MT; i++) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv[i], acc[i][t], 0, 0, 0);
+            }
+        });
+    };
+    U w0[NT], w1[NT];
+    panel_for<0, ITEMS>([&](auto kk) { item(kk, u0, xs0, w0); });
+    for (uint32_t u = u0; u < u1; u += 2) {
+        step(u, xs0, w0, xs1, w1);
+        if (u + 1 < u1) step(u + 1, xs1, w1, xs0, w0);  // uniform
+    }
+    panel_vm_wait();  // no load into LDS outlives the workgroup
+
+    // lane: activation row l % 16 of its tile, weight rows 4 (l / 16) .. + 4
+    const bool quads = a.n % 4 == 0 && ((uintptr_t)(a.part ? (void *)a.part : a.y) & 15) == 0;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t c = n0 + (wave * NT + t) * 16 + 4 * q;
+        if (c >= a.n) continue;
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias && !a.part)
+#pragma unroll
+            for (int v = 0; v < 4; v++) b[v] = c + v < a.n ? round_bf16(a.bias[c + v]) : 0.f;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const uint32_t row = m0 + 16 * i + r;
+            if (row >= a.m) continue;
+            const uint64_t at = (uint64_t)row * a.n + c;
+            f32x4 v = acc[i][t];
+            if (a.part) {
+                float *o = a.part + (uint64_t)part * a.m * a.n + at;
+                if (quads)
+                    *reinterpret_cast<GLOBAL f32x4 *>(gp(o)) = v;
+                else
+                    for (int e = 0; e < 4; e++)
+                        if (c + e < a.n) o[e] = v[e];
+                continue;
+            }
+            const float g = a.inv ? a.inv[row] : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] * g + b[e];
+            if (a.y_bf16) {
+                uint16_t *o = reinterpret_cast<uint16_t *>(a.y) + at;
+                const uint32_t h[4] = {f32_to_bf16_bits(v[0]), f32_to_bf16_bits(v[1]), f32_to_bf16_bits(v[2]), f32_to_bf16_bits(v[3])};
+                if (quads)
+                    *reinterpret_cast<GLOBAL u32x2 *>(gp(o)) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+                else
+                    for (int e = 0; e < 4; e++)
+                        if (c + e < a.n) o[e] = (uint16_t)h[e];
+            } else {
+                float *o = reinterpret_cast<float *>(a.y) + at;
+                if (quads)
+                    *reinterpret_cast<GLOBAL f32x4 *>(gp(o)) = v;
+                else
+                    for (int e = 0; e < 4; e++)
+                        if (c + e < a.n) o[e] = v[e];
+            }
+        }
+    }
+}
+
+typedef void (*PanelFn)(u32x4, u32x4, u32x4, u32x2, PanelArgs);
+
+// The tiles in use: (16-row activation tiles, 16-row weight tiles per
+// wavefront).  Wider ones at eight activation tiles (128 x 128, 128 x 192)
+// leave one wavefront per SIMD with nothing to cover its waits and measured
+// slower than 64 x 192 at every size.
+template <int FMT>
+static PanelFn panel_pick(int mt, int nt) {
+    if (mt == 8) return panel_kernel<FMT, 8, 1>;
+    if (mt == 4) return nt == 3 ? panel_kernel<FMT, 4, 3> : nt == 2 ? panel_kernel<FMT, 4, 2> : panel_kernel<FMT, 4, 1>;
+    return panel_kernel<FMT, 2, 1>;
+}
+
+// Measured per 256 columns (Q4_K, us): a workgroup alone on its CU, and per
+// workgroup with the CU full.  Other formats add their decode per weight tile.
+struct PanelTile {
+    int mt, nt;
+    double alone, full;
+};
+static const PanelTile PANEL_TILES[] = {{4, 3, 3.34, 2.37}, {4, 2, 2.4, 1.8}, {8, 1, 2.1, 2.1}, {4, 1, 1.43, 0.91}, {2, 1, 0.98, 0.55}};
+
+// The tile and the K parts by estimated time, and whether that beats the
+// dequantize pass + GEMM + epilogue.  Both estimates are fits to
+// measurements (Q4_K 12288 x 4096, bf16 out, us, pass and GEMM against this):
+// 32 rows 50.0, 18.2; 64 rows 52.6, 23.7; 128 rows 63.6, 34.7; 256 rows 72.3,
+// 54.2; 512 rows 97, 81.  Q6_K 4096 x 12288: 64 rows 64.7, 33.2; 200 rows
+// 81.1, 70.5; 512 rows 117, 132.  Q8_0 4096 x 4096: 64 rows 22.9, 14.9; 256
+// rows 30.8, 28.7; 512 rows 39.1, 44.  Past a few hundred rows the decode is
+// repeated too often (once per 64 or 128 rows) against one pass for all.
+PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
+    PanelPlan best = {};
+    double decode;
+    switch (format) {
+    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: decode = 0; break;
+    case OCO_Q8_0: case OCO_Q5_K: decode = 0.33; break;
+    case OCO_Q6_K: decode = 0.55; break;
+    default: return best;
+    }
+    const double row_bytes = (double)oco_row_bytes(format, k), passes = 5.1e6;  // bytes per us of the passes over memory
+    if (k % 256 || m == 0 || n == 0 || 192 * row_bytes >= UNIT_OFF || n > 0x3fffffffu || m > 0x3fffffffu) return best;
+    const double mn = (double)m * n, gemm = std::max(k / 512.0, 1.6 * n * k / passes + mn * k / 0.65e9),
+                 vendor = 8 + (n * (2.0 * k + row_bytes) + 4.0 * m * k + 10 * mn) / passes + gemm;
+    const uint32_t units = k / 256;
+    double least = 0.95 * vendor;
+    for (const PanelTile &t : PANEL_TILES)
+        for (uint32_t s = 1; s <= 8 && s <= units; s *= 2) {
+            if (s > 1 && (uint64_t)s * m * 2 > k) break;  // the parts lie where the pass's f16 weights would
+            const double wgs = std::ceil(n / (64.0 * t.nt)) * std::ceil(m / (16.0 * t.mt)) * s;
+            if (wgs >= 2147483647.0) break;
+            const double step = std::max(t.alone + t.nt * decode, wgs / 256 * (t.full + t.nt * decode));
+            const double us = 6 + std::ceil((double)units / s) * step + (s > 1 ? 2.5 + 8.0 * s * mn / passes : 0);
+            if (us < least) {
+                least = us;
+                best = {t.mt, t.nt, s};
+            }
+        }
+    return best;
+}
+
+int panel_launch(uint32_t format, const PanelPlan &pl, const void *w, const uint16_t *x, void *y, bool y_bf16,
+                 const float *bias, const float *inv, float *part, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
+    PanelFn fn = nullptr;
+    switch (format) {
+#define CASE(F) case F: fn = panel_pick<F>(pl.mt, pl.nt); break;
+        CASE(OCO_Q4_0) CASE(OCO_Q4_1) CASE(OCO_Q8_0) CASE(OCO_Q4_K) CASE(OCO_Q5_K) CASE(OCO_Q6_K)
+#undef CASE
+    }
+    if (!fn) return fail(OCO_ERR_UNSUPPORTED, "oco_matmul: format %u", format);
+    PanelArgs a = {};
+    a.w = (const uint8_t *)w;
+    a.x = x;
+    a.n = n;
+    a.k = k;
+    a.m = m;
+    a.row_bytes = (uint32_t)oco_row_bytes(format, k);
+    a.mtiles = (m + 16 * pl.mt - 1) / (16 * pl.mt);
+    a.splits = pl.splits;
+    a.y = y;
+    a.bias = bias;
+    a.inv = inv;
+    a.part = pl.splits > 1 ? part : nullptr;
+    a.y_bf16 = y_bf16;
+    const uint32_t grid = (n + 64 * pl.nt - 1) / (64 * pl.nt) * a.mtiles * pl.splits;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, stream, KPRE_ARGS(a), a);
+    return launch_check("oco_matmul: panel");
+}
+
+}  // namespace oco

@@ -1,0 +1,86 @@
+"""The prompt-chunk GEMM with weights decoded in registers, around the edges
+of its tiles, against the oracle's half-operand product within the
+reference's roundoff bound (matrix_precision.rs:119-142)."""
+import numpy as np
+import pytest
+
+import oracle as O
+import packers as P
+from _util import Guarded, say
+from test_gpu_skinny import product, weights
+
+pytestmark = pytest.mark.gpu
+
+# Shapes of every tile (64 x 192, 64 x 128, 128 x 64, 64 x 64, 32 x 64) with one
+# and several K parts, partial row and column tiles, one to eight 256-column
+# steps (odd and even counts, parts of unequal length).
+SHAPES = [(32, 260, 2304), (33, 1100, 256), (64, 256, 512), (65, 20004, 256), (97, 6144, 1280), (130, 516, 2048),
+          (200, 132, 1280), (257, 8196, 512), (500, 12288, 256)]
+
+
+@pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, P.Q5_K, P.Q6_K, P.Q4_0, P.Q4_1])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_prompt_chunk(lib, fmt, m, n, k):
+    from oco_amd import synth
+    say("prompt chunk", fmt, m, n, k)
+    w = weights(fmt, n, k, 11 + n)
+    x = synth.bf16_bits(synth.activations(12, m * k)).reshape(m, k)
+    rows = np.unique(np.r_[0:8, m // 2:m // 2 + 8, m - 9:m].clip(0, m - 1))
+    half, mag = O.matmul_reference(fmt, w, x[rows], n, k, half_operands=True)
+    got = product(lib, fmt, w, x, m, n, k, offset=7)[rows]
+    assert np.all(np.abs(got - half) <= O.roundoff_bound(half, mag, k, False)), np.abs(got - half).max()
+
+
+@pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, P.Q6_K, P.Q4_1])
+@pytest.mark.parametrize("m,n,k", [(40, 132, 1280), (66, 2052, 256), (257, 8196, 512)])
+def test_prompt_chunk_f16_input_bias_bf16_output(lib, fmt, m, n, k):
+    from oco_amd import synth
+    say("prompt chunk f16", fmt, m, n, k)
+    w = weights(fmt, n, k, 13 + n)
+    x = synth.activations(14, m * k).reshape(m, k).astype(np.float16)
+    bias = np.random.default_rng(m).normal(size=n).astype(np.float32)
+    got = product(lib, fmt, w, x, m, n, k, x_f16=True, y_bf16=True, bias=bias)
+    half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
+    want = half + O.bf16_round(bias)
+    assert np.all(np.abs(got - want) <= O.roundoff_bound(want, mag + np.abs(O.bf16_round(bias)), k, True))
+
+
+def test_prompt_chunk_output_off_its_boundary(lib):
+    """An output that is not 16-byte aligned takes the scalar stores."""
+    from oco_amd import synth
+    m, n, k = 65, 4100, 512
+    w = weights(P.Q4_K, n, k, 23)
+    x = synth.bf16_bits(synth.activations(24, m * k)).reshape(m, k)
+    wb, xb = lib.DeviceBuffer.from_array(w), lib.DeviceBuffer.from_array(x)
+    for dt, size, bits in ((lib.DType.F32, 4, np.uint32), (lib.DType.BF16, 2, np.uint16)):
+        got = []
+        for off in (0, size):
+            y = Guarded(lib, m * n * size + 16)
+            lib.matmul(P.Q4_K, wb, xb, y.ptr + off, lib.Matrix(k, n, m, 0, 1, 1, 0), y_dtype=dt)
+            lib.synchronize()
+            got.append(y.read(np.uint8)[off:off + m * n * size].view(bits))
+        np.testing.assert_array_equal(*got)
+
+
+def test_prompt_chunk_in_graph(lib):
+    """K parts and their sum replay to the eager result."""
+    from oco_amd import synth
+    m, n, k = 48, 1024, 4096
+    w = lib.DeviceBuffer.from_array(weights(P.Q4_K, n, k, 33))
+    x = lib.DeviceBuffer.from_array(synth.bf16_bits(synth.activations(34, m * k)))
+    p, y, eager = lib.Matrix(k, n, m, 0, 1, 1, 0), lib.DeviceBuffer(m * n * 2), lib.DeviceBuffer(m * n * 2)
+    ws = lib.DeviceBuffer(lib.matmul_workspace(P.Q4_K, p))
+    run = lambda out, s=None: lib.matmul(P.Q4_K, w, x, out, p, y_dtype=lib.DType.BF16, stream=s, workspace=ws, workspace_bytes=ws.nbytes)  # noqa: E731
+    s = lib.Stream()
+    g = lib.Graph(s, lambda: run(y, s))
+    run(eager)
+    lib.synchronize()
+    want = eager.download(np.uint16)
+    for _ in range(3):
+        y.fill32(0)
+        lib.synchronize()
+        g.launch()
+        s.sync()
+        np.testing.assert_array_equal(y.download(np.uint16), want)
+        run(eager)
+        lib.synchronize()
