@@ -182,8 +182,11 @@ typedef void (*PanelFn)(u32x4, u32x4, u32x4, u32x2, PanelArgs);
 template <int FMT>
 static PanelFn panel_pick(int mt, int nt) {
     if (mt == 8) return panel_kernel<FMT, 8, 1>;
-    if (mt == 4) return nt == 3 ? panel_kernel<FMT, 4, 3> : nt == 2 ? panel_kernel<FMT, 4, 2> : panel_kernel<FMT, 4, 1>;
-    return panel_kernel<FMT, 2, 1>;
+    if constexpr (FMT == OCO_Q4_K || FMT == OCO_Q4_0 || FMT == OCO_Q4_1) {
+        if (nt == 3) return panel_kernel<FMT, 4, 3>;
+        if (nt == 2) return panel_kernel<FMT, 4, 2>;
+    }
+    return mt == 4 ? panel_kernel<FMT, 4, 1> : panel_kernel<FMT, 2, 1>;
 }
 
 // Measured per 256 columns (Q4_K, us): a workgroup alone on its CU, and per
@@ -216,8 +219,11 @@ PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
     const double mn = (double)m * n, gemm = std::max(k / 512.0, 1.6 * n * k / passes + mn * k / 0.65e9),
                  vendor = 8 + (n * (2.0 * k + row_bytes) + 4.0 * m * k + 10 * mn) / passes + gemm;
     const uint32_t units = k / 256;
-    double least = 0.95 * vendor;
-    for (const PanelTile &t : PANEL_TILES)
+    // Margins for what the fits miss: partial last rounds of workgroups, and
+    // the larger decodes, whose wider tiles also run out of registers.
+    double least = (decode > 0 || m > 512 ? 0.8 : 0.92) * vendor;
+    for (const PanelTile &t : PANEL_TILES) {
+        if (decode > 0 && t.nt > 1) continue;
         for (uint32_t s = 1; s <= 8 && s <= units; s *= 2) {
             if (s > 1 && (uint64_t)s * m * 2 > k) break;  // the parts lie where the pass's f16 weights would
             const double wgs = std::ceil(n / (64.0 * t.nt)) * std::ceil(m / (16.0 * t.mt)) * s;
@@ -229,6 +235,7 @@ PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
                 best = {t.mt, t.nt, s};
             }
         }
+    }
     return best;
 }
 
