@@ -228,7 +228,7 @@ int oco_matvec_relu_sqr(uint32_t format, const void *w, const void *x, oco_dtype
  * `matmul`/`matmul_q4*`/`matmul_tensor_*`, batch.metal:24-79, tensor.metal:9-102).
  * Operands: formats other than MXFP4 decode to f16 (the reference's
  * half(w), tile.metal:16-80) with activations converted to f16; from 32
- * rows (n % 4 == 0) that decode is one pass into a workspace and the
+ * rows that decode is one pass into a workspace and the
  * product a vendor (hipBLASLt) f16 GEMM, below it fused MFMA tiles.  X is
  * bf16 or f16 row-major; Y f32 or bf16.  MXFP4 runs the block-scaled FP6 x
  * FP4 MFMA on the GGUF bytes as stored, with each 32-block of X split into

@@ -659,6 +659,34 @@ __global__ __launch_bounds__(256) void gemm_epilogue_kernel(const float *acc, ui
         *reinterpret_cast<float4 *>(reinterpret_cast<float *>(y) + 4 * i) = make_float4(r[0], r[1], r[2], r[3]);
 }
 
+// The same one element per thread, for outputs whose rows are not whole quads.
+__global__ __launch_bounds__(256) void gemm_epilogue_any_kernel(const float *acc, uint32_t parts, const float *bias,
+                                                                const float *inv_gain, void *y, bool y_bf16, uint32_t n,
+                                                                uint64_t count) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    float r = acc[i];
+    for (uint32_t p = 1; p < parts; p++) r += acc[i + p * count];
+    r = r * (inv_gain ? inv_gain[i / n] : 1.0f) + (bias ? round_bf16(bias[i % n]) : 0.f);
+    if (y_bf16)
+        reinterpret_cast<uint16_t *>(y)[i] = f32_to_bf16_bits(r);
+    else
+        reinterpret_cast<float *>(y)[i] = r;
+}
+
+static int gemm_epilogue_launch(const float *acc, uint32_t parts, const float *bias, const float *inv, void *y, bool y_bf16,
+                                uint32_t m, uint32_t n, hipStream_t stream) {
+    const uint64_t count = (uint64_t)m * n, quads = count / 4;
+    // quads: whole ones per row, in 16-byte accesses
+    if (n % 4 == 0 && ((uintptr_t)y & (y_bf16 ? 7 : 15)) == 0)
+        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, acc, parts,
+                           bias, inv, y, y_bf16, n, quads);
+    else
+        hipLaunchKernelGGL(gemm_epilogue_any_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, acc, parts,
+                           bias, inv, y, y_bf16, n, count);
+    return launch_check("oco_matmul: epilogue");
+}
+
 // One GEMM shape's hipBLASLt objects, built once per (device, m, n, k): D
 // [n rows of m, column-major] = W^T X with W the f16 operands as k x n
 // column-major (the weight rows as stored) and X as k x m.
@@ -813,12 +841,8 @@ static int vendor_matmul(uint32_t format, const void *w, const void *x, oco_dtyp
                                                xo ? (const void *)xo : x, pl.b, &beta, acc, pl.d, acc, pl.d, &pl.algo,
                                                pl.ws ? ws + v.blas : nullptr, pl.ws, stream);
     if (st != HIPBLAS_STATUS_SUCCESS) return fail(OCO_ERR_HIP, "oco_matmul: hipblasLtMatmul status %d", (int)st);
-    if (!direct) {
-        const uint64_t quads = (uint64_t)m * n / 4;
-        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, acc, 1u,
-                           p->has_bias ? bias : nullptr, inv, y, y_dtype == OCO_DT_BF16, n, quads);
-        OCO_TRY(launch_check("oco_matmul: epilogue"));
-    }
+    if (!direct)
+        return gemm_epilogue_launch(acc, 1, p->has_bias ? bias : nullptr, inv, y, y_dtype == OCO_DT_BF16, m, n, stream);
     return OCO_OK;
 }
 
@@ -841,12 +865,7 @@ static int panel_matmul(uint32_t format, const PanelPlan &pp, const void *w, con
     OCO_TRY(launch_check("oco_matmul: f16 activations"));
     const uint16_t *xin = gain || x_dtype == OCO_DT_BF16 ? xo : (const uint16_t *)x;
     OCO_TRY(panel_launch(format, pp, w, xin, y, y_dtype == OCO_DT_BF16, b, inv, part, m, n, k, stream));
-    if (pp.splits > 1) {
-        const uint64_t quads = (uint64_t)m * n / 4;
-        hipLaunchKernelGGL(gemm_epilogue_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, part,
-                           pp.splits, b, inv, y, y_dtype == OCO_DT_BF16, n, quads);
-        OCO_TRY(launch_check("oco_matmul: sum of the parts"));
-    }
+    if (pp.splits > 1) return gemm_epilogue_launch(part, pp.splits, b, inv, y, y_dtype == OCO_DT_BF16, m, n, stream);
     return OCO_OK;
 }
 
@@ -931,13 +950,16 @@ static bool as_matvec(uint32_t format, oco_dtype x_dtype, const oco_matrix *p) {
     return x_dtype == OCO_DT_BF16 && p->m <= vector_rows(format, p->k, p->n) && p->m <= 65535;  // the matvec's row limit
 }
 
-// The vendor path needs n % 4 == 0 (the epilogue's four columns per thread).
 static const BlasPlan *vendor_plan(uint32_t format, oco_dtype x_dtype, const oco_matrix *p) {
-    if (!use_vendor(format, p->m, p->n, x_dtype) || p->n % 4 || p->m == 0 || p->n == 0) return nullptr;
+    if (!use_vendor(format, p->m, p->n, x_dtype) || p->m == 0 || p->n == 0) return nullptr;
     const BlasPlan &pl = blas_plan(p->m, p->n, p->k);
     return pl.ok ? &pl : nullptr;
 }
 
+// Rows that are not whole quads (n % 4 != 0) take the same paths as the
+// others, with the element-wise epilogue: on the fused tiles Q4_K 4098 x 4096
+// took 67 us at 320 rows and 221 at 1000, here 35 and 65.
+//
 // Fewer rows than the dequantize pass pays for go to the few-row kernel,
 // unless an override asks for one of the two paths below it.  (Against the
 // fused tiles, bf16 out, us: Q4_K 12288 x 4096 at 8 rows 52 -> 14.7.)
@@ -979,6 +1001,10 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     const bool aligned = (format != OCO_F16 || ((uintptr_t)w & 15) == 0) &&
                          (x_dtype != OCO_DT_F16 || ((uintptr_t)x & 15) == 0);
     const BlasPlan *pl = aligned ? vendor_plan(format, x_dtype, p) : nullptr;
+    // Rows that are not whole quads ran on the fused tiles without a
+    // workspace: without one they still do.
+    if (pl && p->n % 4 && (!workspace || workspace_bytes < vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws).total))
+        pl = nullptr;
     if (use_skinny(format, p)) {
         const void *xin = x;
         float *inv = nullptr;
@@ -996,6 +1022,12 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     }
     if (pl) {
         const PanelPlan pp = use_panel(format, p);
+        // Odd outputs of short rows: the fused tiles' one launch is the
+        // shorter (Q8_0 2047 x 1024 at 32-1000 rows 16-21 us against 22-23;
+        // at 1700 rows 35 against 31; at k = 4096 55 against 15-25).
+        if (!pp.mt && p->n % 4 && p->k <= 1024 && (uint64_t)p->m * p->n <= 1u << 21 && format != OCO_F16 && format != OCO_F32 &&
+            !q4_gain(format, p->n, x_dtype))
+            return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
         if (pp.mt) {
             const VendorLayout v = vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws);
             OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));

@@ -84,3 +84,28 @@ def test_prompt_chunk_in_graph(lib):
         np.testing.assert_array_equal(y.download(np.uint16), want)
         run(eager)
         lib.synchronize()
+
+
+@pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, P.Q4_0, 0, 1])
+@pytest.mark.parametrize("m,n,k", [(33, 1101, 512), (140, 259, 1280), (520, 134, 256), (64, 130, 1184)])
+def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
+    """n % 4 != 0 from 32 rows on: with the workspace the pass + GEMM or the
+    panel kernel, without it the fused tiles as before; bias, both outputs."""
+    from oco_amd import synth
+    if fmt == P.Q4_K and k % 256:
+        k = 1280
+    say("odd rows", fmt, m, n, k)
+    w = np.frombuffer(np.random.default_rng(n).normal(0, 0.05, n * k).astype(np.float32).tobytes(), np.uint8) if fmt == 0 \
+        else weights(fmt, n, k, 15 + n)
+    x = synth.bf16_bits(synth.activations(16, m * k)).reshape(m, k)
+    bias = np.random.default_rng(m).normal(size=n).astype(np.float32)
+    half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
+    want, size = half + O.bf16_round(bias), mag + np.abs(O.bf16_round(bias))
+    for bf16 in (False, True):
+        got = product(lib, fmt, w, x, m, n, k, y_bf16=bf16, bias=bias)
+        assert np.all(np.abs(got - want) <= O.roundoff_bound(want, size, k, bf16))
+    wb, xb, bb = (lib.DeviceBuffer.from_array(a) for a in (w, x, bias))
+    y, ws = Guarded(lib, m * n * 4), lib.DeviceBuffer(64)
+    lib.matmul(fmt, wb, xb, y.ptr, lib.Matrix(k, n, m, 0, 1, 1, 1), bias=bb, workspace=ws, workspace_bytes=0)
+    lib.synchronize()
+    assert np.all(np.abs(y.read(np.float32).reshape(m, n) - want) <= O.roundoff_bound(want, size, k, False))
