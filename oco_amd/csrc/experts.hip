@@ -4,12 +4,11 @@
 // 107-275) with its kernels expert_expand (projections.metal:78-137),
 // matvec_mxfp4 (:140-182) and moe_sum (routing.metal:157-168).
 //
-// Each workgroup takes one tile of the route plan -- one expert and up to T
-// of the routes that chose it -- and streams that expert's rows once through
-// the LDS tile path of the decode matvec (stream.h), applying every row to
-// all of the tile's routes.  An expert picked by several tokens is therefore
-// read from HBM once per call, not once per route; experts nobody picked are
-// never touched.
+// Each workgroup takes one tile -- a route, or where experts are shared by
+// more routes one expert and up to T of the routes that chose it -- and
+// streams that expert's rows once through the LDS tile path of the decode
+// matvec (stream.h), applying every row to all of the tile's routes.  Experts
+// nobody picked are never touched.
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -82,21 +81,24 @@ __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
     // Which expert and which routes this workgroup serves.
     if (threadIdx.x < 64) {
         if (a.logits) {
+            // the route's token selects; the workgroup of its first route records it
+            const uint32_t y = blockIdx.y, token = y / a.topk, nth = y - token * a.topk;
+            const float *lt = a.logits + (uint64_t)token * a.experts;
             if (a.experts <= 64)
-                select_topk<1>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
+                select_topk<1>(lt, a.experts, a.topk, sel_ids, sel_probs);
+            else if (a.experts <= 128)
+                select_topk<2>(lt, a.experts, a.topk, sel_ids, sel_probs);
             else
-                select_topk<4>(a.logits, a.experts, a.topk, sel_ids, sel_probs);
+                select_topk<4>(lt, a.experts, a.topk, sel_ids, sel_probs);
             __threadfence_block();  // lanes 0 .. topk - 1 wrote the choices
             if (lane == 0) {
-                const uint32_t y = blockIdx.y;
-                tile_meta[0] = sel_ids[y];
+                tile_meta[0] = sel_ids[nth];
                 tile_meta[1] = 1;
                 tile_routes[0] = y;
-                if (blockIdx.x == 0 && blockIdx.y == 0 && a.ids_out)
-                    for (uint32_t r = 0; r < a.topk; r++) {
-                        a.ids_out[r] = sel_ids[r];
-                        a.probs_out[r] = sel_probs[r];
-                    }
+            }
+            if (blockIdx.x == 0 && nth == 0 && a.ids_out && lane < (int)a.topk) {
+                a.ids_out[token * a.topk + lane] = sel_ids[lane];
+                a.probs_out[token * a.topk + lane] = sel_probs[lane];
             }
         } else if (a.desc) {
             // one read: {expert, rows, first sorted row, first list row, route ids}
@@ -104,8 +106,9 @@ __global__ __launch_bounds__(256) void moe_kernel(KPRE_PARAMS, MoeArgs a) {
             if (lane < 2) tile_meta[lane] = v;
             if (lane >= PLAN_DESC_HEAD && lane < PLAN_DESC_HEAD + T) tile_routes[lane - PLAN_DESC_HEAD] = v;
         } else if (lane == 0) {
-            tile_meta[0] = a.ids[blockIdx.y];
-            tile_meta[1] = 1;
+            const uint32_t e = a.ids[blockIdx.y];
+            tile_meta[0] = e;
+            tile_meta[1] = e < a.experts ? 1u : 0u;  // an id past the bank has no rows, as in the route plan
             tile_routes[0] = blockIdx.y;
         }
     }
@@ -359,9 +362,10 @@ static int moe_launch(uint32_t fmt, bool gated, MoeArgs a, uint32_t tiles, uint3
         OCO_TRY(hip_check(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                           "hipFuncSetAttribute"));
     int32_t ov[4];
-    // Three workgroups per CU for MXFP4 banks (gpt-oss B = 1: 33.6 -> 32.4
-    // us against two), two for the others.
-    const uint32_t per_cu = plan_override(OCO_KNOB_MOE_WG, ov) && ov[0] > 0 ? (uint32_t)ov[0] : fmt == OCO_MXFP4 ? 3u : 2u;
+    // Three workgroups per CU for one-route tiles (gpt-oss B = 1: 33.6 -> 32.4
+    // us against two; Q4_K 128 experts, 4 tokens: 52.9 -> 49.7), two for Q8_0
+    // (43.0 against 38.8) and for the wider tiles.
+    const uint32_t per_cu = plan_override(OCO_KNOB_MOE_WG, ov) && ov[0] > 0 ? (uint32_t)ov[0] : t == 1 && fmt != OCO_Q8_0 ? 3u : 2u;
     const uint32_t target = per_cu * device_cus();
     uint32_t gx = std::max<uint32_t>(1, target / std::max<uint32_t>(1, parallel_tiles));
     gx = std::min(gx, a.ngroups);
@@ -471,6 +475,16 @@ static uint8_t *mx_xrec(const oco_experts *w, uint8_t *ws, uint32_t tokens) {
            align256((uint64_t)tokens * w->hidden * 2) + align256((uint64_t)routes * 4) +
            align256((uint64_t)routes * w->hidden * 4);
 }
+
+// Decode batches on the routed kernel: one route per tile, straight from the
+// ids (or the logits), while experts are shared by few routes; tiles of up to
+// MOE_T routes of one expert beyond.  One route needs a quarter of the LDS and
+// about half the registers, so a CU holds more wavefronts, and makes no plan;
+// what it reads twice comes from the caches.  Layer (us; one route, four):
+// Q4_K 128 experts top-8: 4 tokens 50, 66; 8 tokens 74, 108; 16 tokens 121,
+// 203; 64 experts top-8 Q8_0 at 8 tokens 86, 134, at 16 tokens 149, 152; 8
+// experts top-2 Q4_K at 16 tokens 74, 70.
+static bool direct_routes(uint32_t routes, uint32_t experts) { return 2 * (uint64_t)routes <= 3ull * experts; }
 
 static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype, uint32_t *ids, float *probs,
                          const float *logits, uint32_t tokens, uint16_t *out, float *routed, void *workspace,
@@ -649,9 +663,10 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
 
     uint32_t tiles = routes, parallel = routes;
     const uint32_t *tile_desc = nullptr;
-    if (logits && tokens == 1) {
+    const bool direct = tokens == 1 || direct_routes(routes, w->experts);
+    if (logits && direct) {
         // expert_expand (projections.metal:78-137): every gate/up workgroup
-        // selects the token's experts from the logits; workgroup (0, 0)
+        // selects its token's experts from the logits; one workgroup per token
         // records ids and probabilities for the down pass and the combine.
         MoeArgs a = {};
         a.w[0] = (const uint8_t *)w->gate;
@@ -690,7 +705,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
         OCO_TRY(moe_launch(w->format, false, d, routes, routes, s));
         return oco_moe_sum(down, OCO_DT_F32, probs, out, w->hidden, tokens, w->k, stream);
     }
-    if (tokens > 1) {
+    if (!direct) {
         // Tiles of MOE_T routes from descriptors, one workgroup row per slot
         // of their bound.  (The plan's own 16-route tiles, each as four
         // sub-tiles over ceil(routes / 16) + experts slots, made 520 rows of

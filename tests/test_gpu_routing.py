@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from _util import Guarded, say
+from _util import Guarded, rel_l2, say
 
 pytestmark = pytest.mark.gpu
 
@@ -146,3 +146,57 @@ def test_forward_one_token_over_many_experts(lib, fmt, E):
     assert got[0][1][0] == E - 1
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("fmt,tokens,E,k", [(12, 2, 128, 8), (12, 24, 128, 8), (12, 25, 128, 8), (14, 3, 65, 8), (8, 7, 256, 4),
+                                            (39, 3, 32, 4), (12, 31, 8, 2)])
+def test_decode_batches_route_by_route_and_in_tiles(lib, fmt, tokens, E, k):
+    """Up to 1.5 routes per expert every route is a tile of its own and each
+    workgroup selects its token's experts; beyond, tiles of four routes.  Both
+    against the oracle, and the selection against oco_router."""
+    from oco_amd import synth
+    hidden, ffn = 512, 256
+    say("decode batches", fmt, tokens, E, k)
+    host = [synth.weights(fmt, E * n, kk, 80 + i) for i, (n, kk) in enumerate([(ffn, hidden), (ffn, hidden), (hidden, ffn)])]
+    bank = lib.ExpertBank(fmt, hidden, ffn, E, k, *[dev(lib, h) for h in host], activation=1, up_bias_one=False)
+    rng = np.random.default_rng(tokens + E)
+    xs = rng.normal(size=(tokens, hidden)).astype(np.float32)
+    x, rw = dev(lib, xs), dev(lib, (rng.normal(size=(E, hidden)) / 22).astype(np.float32))
+    resid = O.f32_to_bf16(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    out, ids, probs = dev(lib, resid), dev(lib, np.zeros(tokens * k, np.uint32)), lib.DeviceBuffer(tokens * k * 4)
+    routed = Guarded(lib, tokens * k * hidden * 4)
+    bank.forward(rw, None, x, lib.DType.F32, tokens, out, ids, probs, routed=routed.ptr)
+    ids2, probs2 = lib.DeviceBuffer(tokens * k * 4), lib.DeviceBuffer(tokens * k * 4)
+    lib.router(x, lib.DType.F32, rw, None, tokens, hidden, E, k, lib.DeviceBuffer(tokens * E * 4), ids2, probs2)
+    lib.synchronize()
+    got = ids.download(np.uint32).reshape(tokens, k)
+    np.testing.assert_array_equal(got, ids2.download(np.uint32).reshape(tokens, k))
+    np.testing.assert_array_equal(probs.download(np.uint32), probs2.download(np.uint32))
+    ref = O.experts_reference(fmt, hidden, ffn, *host, xs, got, probs.download(np.float32).reshape(tokens, k), resid, activation=1, up_one=False)
+    assert rel_l2(routed.read(np.float32).reshape(-1, hidden), ref["down"]) <= 1e-5
+
+
+@pytest.mark.parametrize("tokens,E", [(2, 64), (20, 16)])
+def test_apply_leaves_out_ids_past_the_bank(lib, tokens, E):
+    """Routes whose id is past the bank have no rows, one route per tile or
+    four; the others' rows are as without them."""
+    from oco_amd import synth
+    hidden, ffn, k = 256, 256, 4
+    say("ids past the bank", tokens, E)
+    bank = lib.ExpertBank(12, hidden, ffn, E, k, *[dev(lib, synth.weights(12, E * 256, 256, 90 + i)) for i in range(3)],
+                          activation=1, up_bias_one=False)
+    rng = np.random.default_rng(tokens)
+    x = dev(lib, rng.normal(size=(tokens, hidden)).astype(np.float32))
+    good = np.stack([rng.permutation(E)[:k] for _ in range(tokens)]).astype(np.uint32)
+    bad = good.copy()
+    bad[1, 2] = E + 1000000
+    probs, rows = dev(lib, np.full((tokens, k), 0.25, np.float32)), []
+    for ids in (good, bad):
+        routed = Guarded(lib, tokens * k * hidden * 4)
+        out = dev(lib, np.zeros((tokens, hidden), np.uint16))
+        bank.apply(x, lib.DType.F32, dev(lib, ids), probs, tokens, out, routed=routed.ptr)
+        lib.synchronize()
+        rows.append(routed.read(np.uint32).reshape(tokens * k, hidden))
+    keep = np.arange(tokens * k) != k + 2
+    np.testing.assert_array_equal(rows[0][keep], rows[1][keep])
+    assert np.all(rows[1][k + 2] == 0x7FC12345)  # untouched
