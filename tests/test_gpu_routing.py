@@ -200,3 +200,24 @@ def test_apply_leaves_out_ids_past_the_bank(lib, tokens, E):
     keep = np.arange(tokens * k) != k + 2
     np.testing.assert_array_equal(rows[0][keep], rows[1][keep])
     assert np.all(rows[1][k + 2] == 0x7FC12345)  # untouched
+
+
+@pytest.mark.parametrize("fmt,ffn,hidden", [(12, 1024, 48 * 16 + 256), (12, 256, 256), (8, 1024, 992), (8, 32, 32), (14, 768, 1280)])
+def test_down_rows_two_at_a_time(lib, fmt, ffn, hidden):
+    """The routed down pass takes two rows per half-wavefront up to 32 pieces
+    a row: the longest such rows, the shortest, and row counts that are not
+    whole groups of sixteen."""
+    from oco_amd import synth
+    E, k, tokens = 16, 2, 3
+    say("down rows", fmt, ffn, hidden)
+    host = [synth.weights(fmt, E * n, kk, 70 + i) for i, (n, kk) in enumerate([(ffn, hidden), (ffn, hidden), (hidden, ffn)])]
+    bank = lib.ExpertBank(fmt, hidden, ffn, E, k, *[dev(lib, h) for h in host], activation=1, up_bias_one=False)
+    rng = np.random.default_rng(ffn + hidden)
+    xs = rng.normal(size=(tokens, hidden)).astype(np.float32)
+    ids, probs = O.select_experts(rng.normal(size=(tokens, E)).astype(np.float32), k)
+    resid = O.f32_to_bf16(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    routed = Guarded(lib, tokens * k * hidden * 4)
+    bank.apply(dev(lib, xs), lib.DType.F32, dev(lib, ids), dev(lib, probs), tokens, dev(lib, resid), routed=routed.ptr)
+    lib.synchronize()
+    ref = O.experts_reference(fmt, hidden, ffn, *host, xs, ids, probs, resid, activation=1, up_one=False)
+    assert rel_l2(routed.read(np.float32).reshape(-1, hidden), ref["down"]) <= 1e-5
