@@ -105,7 +105,7 @@ typedef enum oco_knob {
     OCO_KNOB_STREAM_DIRECT = 11,  /* value 0: Q4_K/Q5_K streaming matvec through the LDS tile even when aligned;
                                      second value (optional): activations 0 staged in LDS, 1 in registers */
     OCO_KNOB_MATMUL_VENDOR = 12,  /* f16-operand prefill: value 0 the fused f16 MFMA tiles, 1 the dequantize pass
-                                     and the vendor GEMM (default: the vendor GEMM from 32 activation rows) */
+                                     and the vendor GEMM (default: by size, among these and the kernels that decode in registers) */
     OCO_KNOB_COUNT = 13
 } oco_knob;
 int oco_plan_override(uint32_t knob, const int32_t *values, uint32_t count);
@@ -227,9 +227,9 @@ int oco_matvec_relu_sqr(uint32_t format, const void *w, const void *x, oco_dtype
  * Replaces DenseMatrix::apply's tiled plans (compute/matrix.rs:130-379,
  * `matmul`/`matmul_q4*`/`matmul_tensor_*`, batch.metal:24-79, tensor.metal:9-102).
  * Operands: formats other than MXFP4 decode to f16 (the reference's
- * half(w), tile.metal:16-80) with activations converted to f16; from 32
- * rows that decode is one pass into a workspace and the
- * product a vendor (hipBLASLt) f16 GEMM, below it fused MFMA tiles.  X is
+ * half(w), tile.metal:16-80) with activations converted to f16: in
+ * registers on the way into the MFMA up to a few hundred rows, for more rows
+ * in one pass into a workspace before a vendor (hipBLASLt) f16 GEMM.  X is
  * bf16 or f16 row-major; Y f32 or bf16.  MXFP4 runs the block-scaled FP6 x
  * FP4 MFMA on the GGUF bytes as stored, with each 32-block of X split into
  * two E2M3 terms with their own E8M0 scales (at most 1/225 of the block

@@ -756,10 +756,11 @@ static bool vendor_format(uint32_t format) {
     return false;
 }
 
-// The vendor path from 32 activation rows, where prefill starts (measured
-// on the box at 32..256 rows: as fast or faster for Q4_K 12288 x 4096, 2-3x
-// for Q8_0 4096 x 4096 and Q6_K 4096 x 12288), unless the
-// OCO_KNOB_MATMUL_VENDOR override chooses.
+// The vendor path's workspace and its products from 32 activation rows on,
+// where the fused tiles fall behind (measured at 32..256 rows: as fast or
+// faster for Q4_K 12288 x 4096, 2-3x for Q8_0 4096 x 4096 and Q6_K 4096 x
+// 12288), unless the OCO_KNOB_MATMUL_VENDOR override chooses; panel_plan
+// (panel.hip) says where decoding in registers is the better choice.
 // The reference scales Q4_0 / Q4_1 activation rows by a power-of-two gain
 // when the matrix has more than 1024 outputs (pipelines.rs:286-288); only
 // the vendor path implements it, so those shapes take it at every tiled m.
