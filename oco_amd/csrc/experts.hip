@@ -456,8 +456,6 @@ uint64_t oco_experts_workspace(const oco_experts *w, uint32_t tokens) {
     uint64_t bytes = align256(oco_route_plan_words((uint32_t)routes, w->experts) * 4) + align256(routes * w->ffn * 4) +
                      align256((uint64_t)tokens * w->hidden * 2) + align256(routes * 4) + align256(routes * w->hidden * 4);
     if (w->format == OCO_Q4_K) bytes += align256(routes * w->ffn * 2);
-    if (w->format != OCO_MXFP4)  // the routed kernel's tile descriptors
-        bytes += align256(plan_desc_words((uint32_t)routes, w->experts, MOE_T) * 4);
     if (w->format == OCO_MXFP4)  // ... and the plan's tile descriptors (tiles of up to 32 rows)
         bytes += align256(mx_rows_bytes(tokens, w->hidden)) + align256(mx_rows_bytes((uint32_t)routes, w->ffn)) +
                  align256(plan_desc_words((uint32_t)routes, w->experts, 32) * 4);
@@ -497,7 +495,13 @@ static uint8_t *mx_xrec(const oco_experts *w, uint8_t *ws, uint32_t tokens) {
 // Q4_K 128 experts top-8: 4 tokens 50, 66; 8 tokens 74, 108; 16 tokens 121,
 // 203; 64 experts top-8 Q8_0 at 8 tokens 86, 134, at 16 tokens 149, 152; 8
 // experts top-2 Q4_K at 16 tokens 74, 70.
-static bool direct_routes(uint32_t routes, uint32_t experts) { return 2 * (uint64_t)routes <= 3ull * experts; }
+// The tiles' descriptors lie where prefill keeps its f16 rows; rows too short
+// to hold them (hidden below 96) take one route per tile too.
+static bool direct_routes(const oco_experts *w, uint32_t tokens) {
+    const uint32_t routes = tokens * w->k;
+    return tokens == 1 || 2 * (uint64_t)routes <= 3ull * w->experts ||
+           plan_desc_words(routes, w->experts, MOE_T) * 4 > align256((uint64_t)tokens * w->hidden * 2);
+}
 
 static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype, uint32_t *ids, float *probs,
                          const float *logits, uint32_t tokens, uint16_t *out, float *routed, void *workspace,
@@ -676,7 +680,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
 
     uint32_t tiles = routes, parallel = routes;
     const uint32_t *tile_desc = nullptr;
-    const bool direct = tokens == 1 || direct_routes(routes, w->experts);
+    const bool direct = direct_routes(w, tokens);
     if (logits && direct) {
         // expert_expand (projections.metal:78-137): every gate/up workgroup
         // selects its token's experts from the logits; one workgroup per token
@@ -724,7 +728,7 @@ static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype,
         // sub-tiles over ceil(routes / 16) + experts slots, made 520 rows of
         // workgroups for the 32 routes of a 4-token batch over 128 experts,
         // nearly all of which read the plan and left: gate/up 42.9 us, down 37.)
-        uint32_t *desc = (uint32_t *)(xrec + (w->format == OCO_Q4_K ? align256((uint64_t)routes * w->ffn * 2) : 0));
+        uint32_t *desc = (uint32_t *)x16;
         PlanSide side = sel;
         side.desc = desc;
         OCO_TRY(route_plan_launch(ids, routes, w->experts, MOE_T, 0, 0, plan, &side, s));
