@@ -190,7 +190,8 @@ static PanelFn panel_pick(int mt, int nt) {
 }
 
 // Measured per 256 columns (Q4_K, us): a workgroup alone on its CU, and per
-// workgroup with the CU full.  Other formats add their decode per weight tile.
+// workgroup with the CU full (weights in the Infinity Cache; streamed from
+// HBM the products of 256 rows and more take about 10% longer on both paths).  Other formats add their decode per weight tile.
 struct PanelTile {
     int mt, nt;
     double alone, full;
@@ -219,16 +220,22 @@ PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
     const double mn = (double)m * n, gemm = std::max(k / 512.0, 1.6 * n * k / passes + mn * k / 0.65e9),
                  vendor = 8 + (n * (2.0 * k + row_bytes) + 4.0 * m * k + 10 * mn) / passes + gemm;
     const uint32_t units = k / 256;
-    // Margins for what the fits miss: partial last rounds of workgroups, and
-    // the larger decodes, whose wider tiles also run out of registers.
-    double least = (decode > 0 || m > 512 ? 0.8 : 0.92) * vendor;
+    // Margins for what the fits miss, the larger decodes and many rows most:
+    // with weights streamed from HBM, 384 rows of Q4_K 12288 x 4096 took 79 us
+    // here against 77, 512 rows 83 against 87.
+    double least = (m > 512 || decode > 0 ? 0.8 : m > 256 ? 0.82 : 0.92) * vendor;
     for (const PanelTile &t : PANEL_TILES) {
         if (decode > 0 && t.nt > 1) continue;
         for (uint32_t s = 1; s <= 8 && s <= units; s *= 2) {
             if (s > 1 && (uint64_t)s * m * 2 > k) break;  // the parts lie where the pass's f16 weights would
             const double wgs = std::ceil(n / (64.0 * t.nt)) * std::ceil(m / (16.0 * t.mt)) * s;
             if (wgs >= 2147483647.0) break;
-            const double step = std::max(t.alone + t.nt * decode, wgs / 256 * (t.full + t.nt * decode));
+            // Past 256 rows: by the fullest CU while two workgroups share it, and
+            // only the widest tile for more (it decodes least per product).
+            double load = wgs / 256;
+            if (m > 256 && load <= 2) load = std::ceil(load);
+            if (m > 256 && load > 2 && t.nt < 3) continue;
+            const double step = std::max(t.alone + t.nt * decode, load * (t.full + t.nt * decode));
             const double us = 6 + std::ceil((double)units / s) * step + (s > 1 ? 2.5 + 8.0 * s * mn / passes : 0);
             if (us < least) {
                 least = us;
