@@ -80,3 +80,38 @@ def test_few_rows_nonfinite_and_rows_apart(lib, fmt):
     keep = [r for r in range(m) if r not in (3, 7)]
     np.testing.assert_array_equal(got[keep], plain[keep])
     np.testing.assert_array_equal(product(lib, fmt, w, x[:5], 5, n, k), plain[:5])
+
+
+@pytest.mark.parametrize("fmt,mid,top", [(P.Q4_0, 8, 15), (P.Q6_K, 32, 63), (P.Q8_0, 0, 127)])
+@pytest.mark.parametrize("m,n,k", [(11, 40, 512), (65, 20004, 256)])  # the few-row kernel; the prompt-chunk GEMM
+def test_infinite_block_scales(lib, fmt, mid, top, m, n, k):
+    """A block's weights are scale * (code - middle): with an infinite scale
+    +-Inf, NaN at the middle code only, whichever kernel decodes it."""
+    from oco_amd import synth
+    say("infinite block scales", fmt, m, n, k)
+    unit, size = (256, 210) if fmt == P.Q6_K else (32, 34 if fmt == P.Q8_0 else 18)
+    w = weights(fmt, n, k, 37).reshape(n, k // unit * size).copy()
+
+    def block(scale_bits, code, first=None):
+        """One block of equal codes, the first of them `first`."""
+        c = np.full(unit, code, np.int64)
+        c[0] = code if first is None else first
+        d = np.array([scale_bits], np.uint16).view(np.uint8)
+        if fmt == P.Q8_0:
+            return np.r_[d, c.astype(np.int8).view(np.uint8)]
+        if fmt == P.Q4_0:
+            return np.r_[d, (c[:16] | (c[16:] << 4)).astype(np.uint8)]
+        q = c.reshape(2, 4, 32)
+        ql = np.concatenate([q[:, :2] & 15 | (q[:, 2:] & 15) << 4], 1).reshape(-1)
+        hi = q >> 4
+        qh = (hi[:, 0] | hi[:, 1] << 2 | hi[:, 2] << 4 | hi[:, 3] << 6).reshape(-1)
+        return np.r_[ql.astype(np.uint8), qh.astype(np.uint8), np.full(16, 3, np.uint8), d]
+
+    inf, ninf, nan = 0x7C00, 0xFC00, 0x7E00
+    w[0, :size], w[1, :size], w[2, :size] = block(inf, top), block(inf, mid - 1), block(inf, top, mid)
+    w[3, :size], w[4, :size], w[5, :size] = block(ninf, mid + 1), block(nan, top), block(inf, mid - 3)
+    x = synth.bf16_bits(np.abs(synth.activations(38, m * k)) + 0.5).reshape(m, k)
+    got = product(lib, fmt, w.reshape(-1), x, m, n, k)
+    want = np.array([np.inf, -np.inf, np.nan, -np.inf, np.nan, -np.inf], np.float32)
+    np.testing.assert_array_equal(got[:, :6], np.broadcast_to(want, (m, 6)))
+    assert np.isfinite(got[:, 6:]).all()
