@@ -239,9 +239,9 @@ int oco_matvec_relu_sqr(uint32_t format, const void *w, const void *x, oco_dtype
  * With bf16 X, up to Builder::dense's vector_rows rows (pipelines.rs:271-283:
  * 1; 4 for Q4_0/Q4_1 and three Q5_K/Q8_0 shapes; 128 for Q8_0 2880 -> 512;
  * every m for F32 with n <= 128) run oco_matvec instead, exact weights and
- * fp32, as DenseMatrix::apply does; Q4_0/Q4_1 with n > 1024 scale each
- * activation row by the reference's power-of-two gain before the f16
- * rounding (matmul_q4_half). */
+ * fp32, as DenseMatrix::apply does; Q4_0/Q4_1 with n > 1024 and n % 4 == 0
+ * scale each activation row by the reference's power-of-two gain before the
+ * f16 rounding (matmul_q4_half). */
 int oco_matmul(uint32_t format, const void *w, const void *x, oco_dtype x_dtype, void *y,
                oco_dtype y_dtype, const float *bias, const oco_matrix *p, oco_stream stream);
 

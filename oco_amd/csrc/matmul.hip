@@ -765,8 +765,10 @@ static bool vendor_format(uint32_t format) {
 // when the matrix has more than 1024 outputs (pipelines.rs:286-288); only
 // the vendor path implements it, so those shapes take it at every tiled m.
 // (f16 activations, which the reference does not take, are used as given.)
+// Rows that are not whole quads run without a workspace too, where there is
+// no place for scaled rows: they take none, with a workspace or without.
 static bool q4_gain(uint32_t format, uint32_t n, oco_dtype x_dtype) {
-    return (format == OCO_Q4_0 || format == OCO_Q4_1) && n > 1024 && x_dtype == OCO_DT_BF16;
+    return (format == OCO_Q4_0 || format == OCO_Q4_1) && n > 1024 && n % 4 == 0 && x_dtype == OCO_DT_BF16;
 }
 
 static bool use_vendor(uint32_t format, uint32_t m, uint32_t n, oco_dtype x_dtype) {

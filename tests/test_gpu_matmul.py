@@ -8,6 +8,8 @@ MXFP4 runs the block-scaled FP6 x FP4 MFMA on the weights as stored, with
 each activation block split into two E2M3 terms: each element is within the
 fp32 roundoff bound plus mx_split_bound, the split's worst case.
 """
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -497,6 +499,57 @@ def test_matmul_q4_row_gain(lib):
             assert np.all(got[r] == 0.0)
             continue
         assert rel_l2(got[r], exact[r]) <= 2e-3
+
+
+@pytest.mark.parametrize("fmt", [P.Q4_0, P.Q4_1])
+@pytest.mark.parametrize("m,gemm", [(5, False), (16, False), (31, False), (40, False), (5, True), (40, True)])
+def test_matmul_q4_row_gain_on_every_route(lib, fmt, m, gemm):
+    """The gain on the few-row kernel, the prompt-chunk GEMM and (asked for)
+    the dequantize pass + GEMM, with bias."""
+    from oco_amd import synth
+    n, k = 1100, 1280
+    say("q4 row gain", fmt, m, gemm)
+    w = synth.weights(fmt, n, k, seed=95)
+    xf = synth.activations(96, m * k).reshape(m, k).astype(np.float64)
+    xf[::3] *= 2.0 ** 20
+    xf[1::3] *= 2.0 ** -30
+    x = synth.bf16_bits(xf.astype(np.float32)).reshape(m, k)
+    bias = np.random.default_rng(m).normal(size=n).astype(np.float32)
+    half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True, row_gain=True)
+    want = half + O.bf16_round(bias)
+    with lib.overridden(lib.Knob.MATMUL_VENDOR, (1,)) if gemm else contextlib.nullcontext():
+        got = run(lib, fmt, w, x, m, n, k, bias=bias)
+    assert np.all(np.abs(got - want) <= O.roundoff_bound(want, mag + np.abs(O.bf16_round(bias)), k, False))
+
+
+@pytest.mark.parametrize("fmt", [P.Q4_0, P.Q4_1])
+@pytest.mark.parametrize("m", [5, 31, 40])
+def test_matmul_q4_odd_rows_take_no_gain(lib, fmt, m):
+    """n > 1024 that is not whole quads: rows are used as given (half(x), Inf
+    past the f16 range), with a workspace and without."""
+    from oco_amd import synth
+    n, k = 1101, 256
+    say("q4 odd rows", fmt, m)
+    w = synth.weights(fmt, n, k, seed=97)
+    xf = synth.activations(98, m * k).reshape(m, k).astype(np.float64)
+    xf[::3] *= 2.0 ** 20
+    xf[1::3] *= 2.0 ** -30
+    x = synth.bf16_bits(xf.astype(np.float32)).reshape(m, k)
+    wb, xb, p = lib.DeviceBuffer.from_array(w), lib.DeviceBuffer.from_array(x), lib.Matrix(k, n, m, 0, 1, 1, 0)
+    with np.errstate(all="ignore"):
+        half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
+        bound = O.roundoff_bound(half, mag, k, False)
+    size = lib.matmul_workspace(fmt, p)
+    for ws, nbytes in ((lib.DeviceBuffer(size + 256), size), (None, 0), (lib.DeviceBuffer(256), 64)):
+        y = Guarded(lib, m * n * 4)
+        lib.matmul(fmt, wb, xb, y.ptr, p, workspace=ws, workspace_bytes=nbytes)
+        lib.synchronize()
+        got = y.read(np.float32).reshape(m, n)
+        big = np.arange(m) % 3 == 0
+        assert not np.isfinite(got[big]).any()
+        assert np.all(got[1::3] == 0.0)  # 2^-30 is below the f16 range
+        rest = np.arange(m) % 3 == 2
+        assert np.all(np.abs(got[rest] - half[rest]) <= bound[rest])
 
 
 @pytest.mark.parametrize("m", [31, 32, 33])
