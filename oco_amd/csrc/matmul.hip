@@ -1003,9 +1003,10 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     // 16-byte aligned for it; otherwise the fused tiles run.
     const bool aligned = (format != OCO_F16 || ((uintptr_t)w & 15) == 0) &&
                          (x_dtype != OCO_DT_F16 || ((uintptr_t)x & 15) == 0);
-    const BlasPlan *pl = aligned ? vendor_plan(format, x_dtype, p) : nullptr;
-    // Rows that are not whole quads ran on the fused tiles without a
-    // workspace: without one they still do.
+    // Rows that are not whole quads need no workspace: without one (and then
+    // without a look at the GEMM library, inside a capture perhaps) they run on
+    // the fused tiles.
+    const BlasPlan *pl = aligned && (p->n % 4 == 0 || workspace) ? vendor_plan(format, x_dtype, p) : nullptr;
     if (pl && p->n % 4 && (!workspace || workspace_bytes < vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws).total))
         pl = nullptr;
     if (use_skinny(format, p)) {
@@ -1048,7 +1049,9 @@ extern "C" int oco_matmul(uint32_t format, const void *w, const void *x, oco_dty
     OCO_TRY(matmul_check(format, w, x, x_dtype, y, y_dtype, bias, p));
     if (p->m == 0 || p->n == 0) return OCO_OK;
     if (as_matvec(format, x_dtype, p)) return oco_matvec(format, w, x, x_dtype, y, y_dtype, bias, nullptr, p, stream);
-    const uint64_t need = oco_matmul_workspace(format, x_dtype, p);
+    // Rows that are not whole quads draw no memory (the pass + GEMM would take
+    // 1.2 GB for 151937 x 4096): they take the paths that need no workspace.
+    const uint64_t need = p->n % 4 && !use_mx(format) ? 0 : oco_matmul_workspace(format, x_dtype, p);
     if (!need) return oco_matmul_ws(format, w, x, x_dtype, y, y_dtype, bias, p, nullptr, 0, stream);
     void *ws = nullptr;
     OCO_TRY(hip_check(hipMallocAsync(&ws, need, (hipStream_t)stream), "oco_matmul: hipMallocAsync"));

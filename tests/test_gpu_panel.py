@@ -1,6 +1,8 @@
 """The prompt-chunk GEMM with weights decoded in registers, around the edges
 of its tiles, against the oracle's half-operand product within the
 reference's roundoff bound (matrix_precision.rs:119-142)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -86,6 +88,47 @@ def test_prompt_chunk_in_graph(lib):
         lib.synchronize()
 
 
+def pool_high_water(reset=False):
+    """Most bytes drawn at once from the device's stream-ordered pool."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip, pool, value = ctypes.CDLL(path), ctypes.c_void_p(), ctypes.c_uint64(0)
+    assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+    used_mem_high = 8  # hipMemPoolAttrUsedMemHigh
+    if reset:
+        assert hip.hipMemPoolSetAttribute(pool, used_mem_high, ctypes.byref(value)) == 0
+    assert hip.hipMemPoolGetAttribute(pool, used_mem_high, ctypes.byref(value)) == 0
+    return value.value
+
+
+@pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, 1])
+def test_odd_rows_without_a_workspace_draw_no_memory(lib, fmt):
+    """oco_matmul with n % 4 != 0 takes nothing from the stream-ordered pool
+    (whole quads do), and its launch can be recorded and replayed."""
+    from oco_amd import synth
+    m, k = 40, 512
+    say("odd rows draw no memory", fmt)
+    x = lib.DeviceBuffer.from_array(synth.bf16_bits(synth.activations(36, m * k)))
+    drawn = []
+    for n in (1101, 1104):
+        w, y = lib.DeviceBuffer.from_array(weights(fmt, n, k, 35)), lib.DeviceBuffer(m * n * 4)
+        p = lib.Matrix(k, n, m, 0, 1, 1, 0)
+        lib.synchronize()
+        pool_high_water(reset=True)
+        lib.matmul(fmt, w, x, y, p)
+        lib.synchronize()
+        drawn.append(pool_high_water())
+        if n % 4:
+            s, z = lib.Stream(), lib.DeviceBuffer(m * n * 4)
+            g = lib.Graph(s, lambda: lib.matmul(fmt, w, x, z, p, stream=s))
+            for _ in range(2):
+                z.fill32(0)
+                lib.synchronize()
+                g.launch()
+                s.sync()
+                np.testing.assert_array_equal(z.download(np.uint32), y.download(np.uint32))
+    assert drawn[0] == 0 and drawn[1] > 0
+
+
 @pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, P.Q4_0, 0, 1])
 @pytest.mark.parametrize("m,n,k", [(33, 1101, 512), (140, 259, 1280), (520, 134, 256), (64, 130, 1184)])
 def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
@@ -102,7 +145,7 @@ def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
     half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
     want, size = half + O.bf16_round(bias), mag + np.abs(O.bf16_round(bias))
     for bf16 in (False, True):
-        got = product(lib, fmt, w, x, m, n, k, y_bf16=bf16, bias=bias)
+        got = product(lib, fmt, w, x, m, n, k, y_bf16=bf16, bias=bias, workspace=True)
         assert np.all(np.abs(got - want) <= O.roundoff_bound(want, size, k, bf16))
     wb, xb, bb = (lib.DeviceBuffer.from_array(a) for a in (w, x, bias))
     y, ws = Guarded(lib, m * n * 4), lib.DeviceBuffer(64)

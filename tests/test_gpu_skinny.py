@@ -20,12 +20,14 @@ def weights(fmt, n, k, seed):
     return synth.weights(fmt, n, k, seed=seed)
 
 
-def product(lib, fmt, w, x, m, n, k, x_f16=False, y_bf16=False, bias=None, offset=0):
+def product(lib, fmt, w, x, m, n, k, x_f16=False, y_bf16=False, bias=None, offset=0, workspace=False):
     keep, wp = upload_at_offset(lib, w, offset)
     xb, bb = lib.DeviceBuffer.from_array(x), None if bias is None else lib.DeviceBuffer.from_array(bias)
     y = Guarded(lib, m * n * (2 if y_bf16 else 4))
-    lib.matmul(fmt, wp, xb, y.ptr, lib.Matrix(k, n, m, 0, 1, 1, 0 if bias is None else 1),
-               lib.DType.F16 if x_f16 else lib.DType.BF16, lib.DType.BF16 if y_bf16 else lib.DType.F32, bb)
+    p, xt = lib.Matrix(k, n, m, 0, 1, 1, 0 if bias is None else 1), lib.DType.F16 if x_f16 else lib.DType.BF16
+    need = lib.matmul_workspace(fmt, p, xt) if workspace else 0
+    lib.matmul(fmt, wp, xb, y.ptr, p, xt, lib.DType.BF16 if y_bf16 else lib.DType.F32, bb,
+               workspace=lib.DeviceBuffer(need) if need else None, workspace_bytes=need)
     lib.synchronize()
     got = y.read(np.uint16 if y_bf16 else np.float32)
     return (O.bf16_to_f32(got) if y_bf16 else got).reshape(m, n)
