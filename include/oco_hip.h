@@ -105,7 +105,8 @@ typedef enum oco_knob {
     OCO_KNOB_STREAM_DIRECT = 11,  /* value 0: Q4_K/Q5_K streaming matvec through the LDS tile even when aligned;
                                      second value (optional): activations 0 staged in LDS, 1 in registers */
     OCO_KNOB_MATMUL_VENDOR = 12,  /* f16-operand prefill: value 0 the fused f16 MFMA tiles, 1 the dequantize pass
-                                     and the vendor GEMM (default: by size, among these and the kernels that decode in registers) */
+                                     and the vendor GEMM, 2 with row tiles, column tiles and K parts the panel
+                                     kernel (default: by size, among these and the few-row kernel) */
     OCO_KNOB_COUNT = 13
 } oco_knob;
 int oco_plan_override(uint32_t knob, const int32_t *values, uint32_t count);
@@ -254,6 +255,22 @@ uint64_t oco_matmul_workspace(uint32_t format, oco_dtype x_dtype, const oco_matr
 int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_dtype x_dtype, void *y,
                   oco_dtype y_dtype, const float *bias, const oco_matrix *p, void *workspace,
                   uint64_t workspace_bytes, oco_stream stream);
+
+/* The kernel oco_matmul_ws takes for this call, 16-byte aligned operands and a
+ * workspace of this size (0: none) given: route[0] an oco_matmul_kernel and,
+ * for the panel kernel, route[1..3] its 16-row activation tiles, 16-row weight
+ * tiles per wavefront and K parts (else 0).  No counterpart in the reference;
+ * for tests and tuning, like oco_plan_override. */
+typedef enum oco_matmul_kernel {
+    OCO_MATMUL_VECTOR = 0,   /* the decode matvec on each row */
+    OCO_MATMUL_MX = 1,       /* MXFP4: the block-scaled MFMA */
+    OCO_MATMUL_FEW_ROWS = 2, /* weights decoded in registers, K split over a workgroup's wavefronts */
+    OCO_MATMUL_TILES = 3,    /* fused f16 MFMA tiles, weights decoded into LDS */
+    OCO_MATMUL_PANEL = 4,    /* prompt chunks, weights decoded in registers */
+    OCO_MATMUL_GEMM = 5      /* dequantize pass, then the vendor GEMM */
+} oco_matmul_kernel;
+int oco_matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, uint64_t workspace_bytes,
+                     uint32_t route[4]);
 
 /* The norm -> MXFP4 prefill pair in two launches instead of three: the RMS
  * norm of oco_norm (same rounding) whose workgroups also split each output

@@ -966,16 +966,75 @@ static const BlasPlan *vendor_plan(uint32_t format, oco_dtype x_dtype, const oco
 // Fewer rows than the dequantize pass pays for go to the few-row kernel,
 // unless an override asks for one of the two paths below it.  (Against the
 // fused tiles, bf16 out, us: Q4_K 12288 x 4096 at 8 rows 52 -> 14.7.)
-static bool use_skinny(uint32_t format, const oco_matrix *p) {
+static bool matmul_override() {
     int32_t ov[4];
-    return p->m < 32 && !plan_override(OCO_KNOB_MATMUL_VENDOR, ov) && !plan_override(OCO_KNOB_MATMUL_TILE, ov) &&
-           skinny_fits(format, p->m, p->n, p->k);
+    return plan_override(OCO_KNOB_MATMUL_VENDOR, ov) || plan_override(OCO_KNOB_MATMUL_TILE, ov);
 }
 
-static PanelPlan use_panel(uint32_t format, const oco_matrix *p) {
+static bool use_skinny(uint32_t format, const oco_matrix *p) {
+    return p->m < 32 && !matmul_override() && skinny_fits(format, p->m, p->n, p->k);
+}
+
+// Odd outputs of short rows: the fused tiles' one launch is the shorter
+// (Q8_0 2047 x 1024 at 32-1000 rows 16-21 us against 22-23; at 1700 rows 35
+// against 31; at k = 4096 55 against 15-25).
+static bool use_short_rows(uint32_t format, const oco_matrix *p, bool panel) {
+    return !panel && p->n % 4 && p->k <= 1024 && (uint64_t)p->m * p->n <= 1u << 21 && format != OCO_F16 && format != OCO_F32;
+}
+
+// The kernel a checked product takes (not the matvec, not MXFP4), and what it
+// was chosen with: the GEMM's plan (null: no workspace) and the panel's tile.
+struct Route {
+    oco_matmul_kernel kernel;
+    const BlasPlan *pl;
+    PanelPlan panel;
+};
+
+static int matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, bool aligned, bool workspace,
+                        uint64_t workspace_bytes, Route *r) {
+    *r = {OCO_MATMUL_TILES, nullptr, {}};
+    // Rows that are not whole quads need no workspace: without one (and then
+    // without a look at the GEMM library, inside a capture perhaps) they run on
+    // the fused tiles.
+    if (aligned && (p->n % 4 == 0 || workspace)) r->pl = vendor_plan(format, x_dtype, p);
+    if (r->pl && p->n % 4 && workspace_bytes < vendor_layout(format, x_dtype, p->m, p->n, p->k, r->pl->ws).total) r->pl = nullptr;
+    if (use_skinny(format, p)) {
+        r->kernel = OCO_MATMUL_FEW_ROWS;
+        return OCO_OK;
+    }
+    if (!r->pl) return OCO_OK;
     int32_t ov[4];
-    if (plan_override(OCO_KNOB_MATMUL_VENDOR, ov) || plan_override(OCO_KNOB_MATMUL_TILE, ov)) return {};
-    return panel_plan(format, p->m, p->n, p->k);
+    const uint32_t set = plan_override(OCO_KNOB_MATMUL_VENDOR, ov);
+    if (set && ov[0] == 2) {  // the panel kernel, with this tile
+        r->panel = {set > 1 ? ov[1] : 0, set > 2 ? ov[2] : 0, set > 3 ? (uint32_t)ov[3] : 1};
+        if (!panel_fits(format, r->panel, p->m, p->n, p->k))
+            return fail(OCO_ERR_INVALID, "oco_matmul: no panel tile %d x %d in %u parts for format %u, %u x %u x %u", r->panel.mt,
+                        r->panel.nt, r->panel.splits, format, p->m, p->n, p->k);
+        r->kernel = OCO_MATMUL_PANEL;
+        return OCO_OK;
+    }
+    if (!matmul_override()) {
+        r->panel = panel_plan(format, p->m, p->n, p->k);
+        if (use_short_rows(format, p, r->panel.mt != 0)) return OCO_OK;
+    }
+    r->kernel = r->panel.mt ? OCO_MATMUL_PANEL : OCO_MATMUL_GEMM;
+    return OCO_OK;
+}
+
+extern "C" int oco_matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, uint64_t workspace_bytes,
+                                uint32_t route[4]) {
+    if (!p || !route) return fail(OCO_ERR_INVALID, "oco_matmul_route: null argument");
+    Route r = {OCO_MATMUL_VECTOR, nullptr, {}};
+    if (use_mx(format) && !as_matvec(format, x_dtype, p))
+        r.kernel = OCO_MATMUL_MX;
+    else if (!as_matvec(format, x_dtype, p))
+        OCO_TRY(matmul_route(format, x_dtype, p, true, workspace_bytes != 0, workspace_bytes, &r));
+    const bool panel = r.kernel == OCO_MATMUL_PANEL;
+    route[0] = r.kernel;
+    route[1] = panel ? r.panel.mt : 0;
+    route[2] = panel ? r.panel.nt : 0;
+    route[3] = panel ? r.panel.splits : 0;
+    return OCO_OK;
 }
 
 extern "C" uint64_t oco_matmul_workspace(uint32_t format, oco_dtype x_dtype, const oco_matrix *p) {
@@ -1003,13 +1062,10 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     // 16-byte aligned for it; otherwise the fused tiles run.
     const bool aligned = (format != OCO_F16 || ((uintptr_t)w & 15) == 0) &&
                          (x_dtype != OCO_DT_F16 || ((uintptr_t)x & 15) == 0);
-    // Rows that are not whole quads need no workspace: without one (and then
-    // without a look at the GEMM library, inside a capture perhaps) they run on
-    // the fused tiles.
-    const BlasPlan *pl = aligned && (p->n % 4 == 0 || workspace) ? vendor_plan(format, x_dtype, p) : nullptr;
-    if (pl && p->n % 4 && (!workspace || workspace_bytes < vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws).total))
-        pl = nullptr;
-    if (use_skinny(format, p)) {
+    Route r;
+    OCO_TRY(matmul_route(format, x_dtype, p, aligned, workspace != nullptr, workspace_bytes, &r));
+    const BlasPlan *pl = r.pl;
+    if (r.kernel == OCO_MATMUL_FEW_ROWS) {
         const void *xin = x;
         float *inv = nullptr;
         if (pl && q4_gain(format, p->n, x_dtype)) {  // scaled f16 rows through the workspace, as the vendor path makes them
@@ -1024,24 +1080,13 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
         return skinny_launch(format, w, xin, x_dtype == OCO_DT_F16 || inv, y, y_dtype == OCO_DT_BF16, p->has_bias ? bias : nullptr,
                              inv, p->m, p->n, p->k, (hipStream_t)stream);
     }
-    if (pl) {
-        const PanelPlan pp = use_panel(format, p);
-        // Odd outputs of short rows: the fused tiles' one launch is the
-        // shorter (Q8_0 2047 x 1024 at 32-1000 rows 16-21 us against 22-23;
-        // at 1700 rows 35 against 31; at k = 4096 55 against 15-25).
-        if (!pp.mt && p->n % 4 && p->k <= 1024 && (uint64_t)p->m * p->n <= 1u << 21 && format != OCO_F16 && format != OCO_F32 &&
-            !q4_gain(format, p->n, x_dtype))
-            return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
-        if (pp.mt) {
-            const VendorLayout v = vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws);
-            OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));
-            return panel_matmul(format, pp, w, x, x_dtype, y, y_dtype, bias, p, v, workspace, (hipStream_t)stream);
-        }
+    if (r.kernel == OCO_MATMUL_TILES) return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
+    if (r.kernel == OCO_MATMUL_PANEL) {
+        const VendorLayout v = vendor_layout(format, x_dtype, p->m, p->n, p->k, pl->ws);
+        OCO_TRY(vendor_workspace_check(workspace, workspace_bytes, v.total));
+        return panel_matmul(format, r.panel, w, x, x_dtype, y, y_dtype, bias, p, v, workspace, (hipStream_t)stream);
     }
-    if (pl)
-        return vendor_matmul(format, w, x, x_dtype, y, y_dtype, bias, p, *pl, workspace, workspace_bytes,
-                             (hipStream_t)stream);
-    return matmul_decode_launch(format, w, x, x_dtype, y, y_dtype, bias, p, (hipStream_t)stream);
+    return vendor_matmul(format, w, x, x_dtype, y, y_dtype, bias, p, *pl, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int oco_matmul(uint32_t format, const void *w, const void *x, oco_dtype x_dtype, void *y,

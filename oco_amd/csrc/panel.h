@@ -14,6 +14,9 @@ struct PanelPlan {
     uint32_t splits;
 };
 PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k);
+// Whether a tile and K parts can run: a tile built for the format, offsets
+// within 32 bits, and the f32 parts within the f16 weights' place.
+bool panel_fits(uint32_t format, const PanelPlan &pl, uint32_t m, uint32_t n, uint32_t k);
 
 // x: f16 rows, 16-byte aligned.  With pl.splits > 1 the f32 parts go to
 // part[splits][m][n] and the caller sums them; else y = X W^T (times

@@ -198,6 +198,28 @@ struct PanelTile {
 };
 static const PanelTile PANEL_TILES[] = {{4, 3, 3.34, 2.37}, {4, 2, 2.4, 1.8}, {8, 1, 2.1, 2.1}, {4, 1, 1.43, 0.91}, {2, 1, 0.98, 0.55}};
 
+// us per 256 columns and weight tile that a format's decode adds; below zero:
+// not decoded here.
+static double panel_decode(uint32_t format) {
+    switch (format) {
+    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: return 0;
+    case OCO_Q8_0: case OCO_Q5_K: return 0.33;
+    case OCO_Q6_K: return 0.55;
+    }
+    return -1;
+}
+
+bool panel_fits(uint32_t format, const PanelPlan &pl, uint32_t m, uint32_t n, uint32_t k) {
+    const double decode = panel_decode(format);
+    if (decode < 0 || k == 0 || k % 256 || m == 0 || n == 0 || m > 0x3fffffffu || n > 0x3fffffffu) return false;
+    bool built = false;
+    for (const PanelTile &t : PANEL_TILES) built = built || (t.mt == pl.mt && t.nt == pl.nt && (t.nt == 1 || decode == 0));
+    if (!built || 64ull * pl.nt * oco_row_bytes(format, k) >= UNIT_OFF) return false;
+    const uint64_t s = pl.splits;
+    if (s == 0 || s > k / 256 || (s > 1 && s * m * 2 > k)) return false;  // the parts lie where the pass's f16 weights would
+    return (uint64_t)((n + 64 * pl.nt - 1) / (64 * pl.nt)) * ((m + 16 * pl.mt - 1) / (16 * pl.mt)) * s < 0x80000000ull;
+}
+
 // The tile and the K parts by estimated time, and whether that beats the
 // dequantize pass + GEMM + epilogue.  Both estimates are fits to
 // measurements (Q4_K 12288 x 4096, bf16 out, us, pass and GEMM against this):
@@ -208,15 +230,9 @@ static const PanelTile PANEL_TILES[] = {{4, 3, 3.34, 2.37}, {4, 2, 2.4, 1.8}, {8
 // repeated too often (once per 64 or 128 rows) against one pass for all.
 PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
     PanelPlan best = {};
-    double decode;
-    switch (format) {
-    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: decode = 0; break;
-    case OCO_Q8_0: case OCO_Q5_K: decode = 0.33; break;
-    case OCO_Q6_K: decode = 0.55; break;
-    default: return best;
-    }
+    const double decode = panel_decode(format);
+    if (!panel_fits(format, {2, 1, 1}, m, n, k)) return best;
     const double row_bytes = (double)oco_row_bytes(format, k), passes = 5.1e6;  // bytes per us of the passes over memory
-    if (k % 256 || m == 0 || n == 0 || 192 * row_bytes >= UNIT_OFF || n > 0x3fffffffu || m > 0x3fffffffu) return best;
     const double mn = (double)m * n, gemm = std::max(k / 512.0, 1.6 * n * k / passes + mn * k / 0.65e9),
                  vendor = 8 + (n * (2.0 * k + row_bytes) + 4.0 * m * k + 10 * mn) / passes + gemm;
     const uint32_t units = k / 256;
@@ -225,11 +241,9 @@ PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
     // here against 77, 512 rows 83 against 87.
     double least = (m > 512 || decode > 0 ? 0.8 : m > 256 ? 0.82 : 0.92) * vendor;
     for (const PanelTile &t : PANEL_TILES) {
-        if (decode > 0 && t.nt > 1) continue;
-        for (uint32_t s = 1; s <= 8 && s <= units; s *= 2) {
-            if (s > 1 && (uint64_t)s * m * 2 > k) break;  // the parts lie where the pass's f16 weights would
+        for (uint32_t s = 1; s <= 8; s *= 2) {
+            if (!panel_fits(format, {t.mt, t.nt, s}, m, n, k)) break;
             const double wgs = std::ceil(n / (64.0 * t.nt)) * std::ceil(m / (16.0 * t.mt)) * s;
-            if (wgs >= 2147483647.0) break;
             // Past 256 rows: by the fullest CU while two workgroups share it, and
             // only the widest tile for more (it decodes least per product).
             double load = wgs / 256;

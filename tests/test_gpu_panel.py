@@ -13,9 +13,8 @@ from test_gpu_skinny import product, weights
 
 pytestmark = pytest.mark.gpu
 
-# Shapes of every tile (64 x 192, 64 x 128, 128 x 64, 64 x 64, 32 x 64) with one
-# and several K parts, partial row and column tiles, one to eight 256-column
-# steps (odd and even counts, parts of unequal length).
+# Partial row and column tiles, one to nine 256-column steps, on whichever
+# kernel the choice takes; test_every_tile pins the tile and the K parts.
 SHAPES = [(32, 260, 2304), (33, 1100, 256), (64, 256, 512), (65, 20004, 256), (97, 6144, 1280), (130, 516, 2048),
           (200, 132, 1280), (257, 8196, 512), (500, 12288, 256)]
 
@@ -31,6 +30,55 @@ def test_prompt_chunk(lib, fmt, m, n, k):
     half, mag = O.matmul_reference(fmt, w, x[rows], n, k, half_operands=True)
     got = product(lib, fmt, w, x, m, n, k, offset=7)[rows]
     assert np.all(np.abs(got - half) <= O.roundoff_bound(half, mag, k, False)), np.abs(got - half).max()
+
+
+Q4 = (P.Q4_0, P.Q4_1, P.Q4_K)  # the formats of the wider tiles
+TILES = [(fmt, mt, nt) for fmt in (P.Q8_0, P.Q4_K, P.Q5_K, P.Q6_K, P.Q4_0, P.Q4_1)
+         for mt, nt in [(2, 1), (4, 1), (8, 1), (4, 2), (4, 3)] if nt == 1 or fmt in Q4]
+
+
+@pytest.mark.parametrize("fmt,mt,nt", TILES)
+def test_every_tile(lib, fmt, mt, nt):
+    """Each tile of each format (16 mt activation rows x 64 nt weight rows),
+    pinned: one K part over an odd and an even number of 256-column steps and
+    over one; two and four parts of unequal length; rows and columns one past
+    and one short of whole tiles; rows that are not whole quads with one part
+    and with several; f32 and bf16 outputs, bias, f16 activations."""
+    from oco_amd import synth
+    rows, cols = 16 * mt, 64 * nt
+    for parts, m, n, k, options in [
+            (1, rows + 1, cols + 4, 768, {}), (1, 2 * rows - 1, 2 * cols - 4, 512, dict(y_bf16=True)),
+            (1, rows, cols, 256, dict(x_f16=True)), (1, 3 * rows - 5, cols + 1, 1024, dict(workspace=True)),
+            (2, rows + 1, cols + 4, 768, dict(y_bf16=True)), (4, rows - 1, 2 * cols, 1280, {}),
+            (4, rows + 3, cols - 1, 1280, dict(workspace=True)), (3, 2, 3 * cols + 3, 1024, dict(workspace=True, x_f16=True))]:
+        say("tile", fmt, mt, nt, parts, m, n, k, options)
+        w = weights(fmt, n, k, 51 + n)
+        x = synth.activations(52, m * k).reshape(m, k)
+        f16 = options.get("x_f16", False)
+        x = x.astype(np.float16) if f16 else synth.bf16_bits(x).reshape(m, k)
+        bias = np.random.default_rng(m + n).normal(size=n).astype(np.float32)
+        half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
+        want = half + O.bf16_round(bias)
+        with lib.overridden(lib.Knob.MATMUL_VENDOR, (2, mt, nt, parts)):
+            route = lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 1), lib.DType.F16 if f16 else lib.DType.BF16)
+            assert route == (lib.MatmulKernel.PANEL, mt, nt, parts)
+            got = product(lib, fmt, w, x, m, n, k, bias=bias, offset=5, **options)
+        bound = O.roundoff_bound(want, mag + np.abs(O.bf16_round(bias)), k, options.get("y_bf16", False))
+        assert np.all(np.abs(got - want) <= bound), (parts, m, n, k, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("fmt,values,m,k", [(P.Q4_K, (2, 3, 1, 1), 64, 512), (P.Q8_0, (2, 4, 2, 1), 64, 512), (P.Q4_K, (2, 4, 1, 3), 40, 512),
+                                            (P.Q4_K, (2, 4, 1, 2), 200, 512), (P.Q4_K, (2, 4, 1, 0), 64, 512), (P.Q4_K, (2,), 64, 512),
+                                            (P.Q8_0, (2, 4, 1, 1), 64, 288), (1, (2, 4, 1, 1), 64, 512)])
+def test_a_pinned_tile_that_cannot_run_is_refused(lib, fmt, values, m, k):
+    """A tile that is not built, more parts than 256-column steps or than the
+    workspace holds, no parts, a K that is not whole steps, another format."""
+    say("tile refused", fmt, values, m, k)
+    p, y = lib.Matrix(k, 128, m, 0, 1, 1, 0), lib.DeviceBuffer(m * 128 * 4)
+    w, x = lib.DeviceBuffer.from_array(weights(fmt, 128, k, 61)), lib.DeviceBuffer(m * k * 2)
+    with lib.overridden(lib.Knob.MATMUL_VENDOR, values):
+        with pytest.raises(lib.OcoError, match="no panel tile"):
+            lib.matmul(fmt, w, x, y, p)
 
 
 @pytest.mark.parametrize("fmt", [P.Q8_0, P.Q4_K, P.Q6_K, P.Q4_1])
@@ -152,3 +200,4 @@ def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
     lib.matmul(fmt, wb, xb, y.ptr, lib.Matrix(k, n, m, 0, 1, 1, 1), bias=bb, workspace=ws, workspace_bytes=0)
     lib.synchronize()
     assert np.all(np.abs(y.read(np.float32).reshape(m, n) - want) <= O.roundoff_bound(want, size, k, False))
+

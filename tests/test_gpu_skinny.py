@@ -26,8 +26,8 @@ def product(lib, fmt, w, x, m, n, k, x_f16=False, y_bf16=False, bias=None, offse
     y = Guarded(lib, m * n * (2 if y_bf16 else 4))
     p, xt = lib.Matrix(k, n, m, 0, 1, 1, 0 if bias is None else 1), lib.DType.F16 if x_f16 else lib.DType.BF16
     need = lib.matmul_workspace(fmt, p, xt) if workspace else 0
-    lib.matmul(fmt, wp, xb, y.ptr, p, xt, lib.DType.BF16 if y_bf16 else lib.DType.F32, bb,
-               workspace=lib.DeviceBuffer(need) if need else None, workspace_bytes=need)
+    ws = lib.DeviceBuffer(need) if need else None
+    lib.matmul(fmt, wp, xb, y.ptr, p, xt, lib.DType.BF16 if y_bf16 else lib.DType.F32, bb, workspace=ws, workspace_bytes=need)
     lib.synchronize()
     got = y.read(np.uint16 if y_bf16 else np.float32)
     return (O.bf16_to_f32(got) if y_bf16 else got).reshape(m, n)
