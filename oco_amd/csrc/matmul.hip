@@ -975,11 +975,28 @@ static bool use_skinny(uint32_t format, const oco_matrix *p) {
     return p->m < 32 && !matmul_override() && skinny_fits(format, p->m, p->n, p->k);
 }
 
-// Odd outputs of short rows: the fused tiles' one launch is the shorter
-// (Q8_0 2047 x 1024 at 32-1000 rows 16-21 us against 22-23; at 1700 rows 35
-// against 31; at k = 4096 55 against 15-25).
+// Rows that are not whole quads over a short K: the fused tiles' one launch
+// against the panel kernel's two or three and the pass + GEMM's.  The fused
+// tiles' time is their K steps while they fill the chip once, the GEMM's grows
+// with the outputs.  (us; fused, then panel or GEMM; weights from HBM.)
+//   k = 256:  Q8_0 2047 at 1000 rows 8.4, panel 13.0; 8191 at 200 rows 8.9,
+//             panel 12.2, at 1000 rows 33.6, GEMM 46; Q6_K 38.5, 48.1
+//   k = 512:  Q8_0 2047 at 300 rows 11.3, GEMM 14.9; 4097 at 1000 rows 44, 31
+//   k = 1024: Q8_0 515 at 300 rows 18.6, GEMM 14.3; 2047 at 300 rows 19.0,
+//             17.5, at 1000 rows 20.9, 26.7; Q4_K 4097 at 300 rows 21.4, 24.8;
+//             Q6_K 26.0, 24.8
+// Q4 formats: the panel kernel, where it is chosen, is mostly the shorter
+// (8191 x 256 at 1000 rows 33.7, 27.7; 2047 x 256 9.1, 10.3).  Q5_K's fused
+// decode never is (2047 x 512 at 300 rows 47, GEMM 19).
 static bool use_short_rows(uint32_t format, const oco_matrix *p, bool panel) {
-    return !panel && p->n % 4 && p->k <= 1024 && (uint64_t)p->m * p->n <= 1u << 21 && format != OCO_F16 && format != OCO_F32;
+    const uint64_t mn = (uint64_t)p->m * p->n;
+    if (p->n % 4 == 0 || p->k > 1024 || mn > (p->k <= 256 ? 1u << 24 : 1u << 21) || (p->k > 512 && mn < 15u << 16)) return false;
+    switch (format) {
+    case OCO_Q8_0: return p->k <= 256 || !panel;
+    case OCO_Q6_K: return p->k <= 256 || (p->k <= 512 && !panel);
+    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: return !panel;
+    }
+    return false;
 }
 
 // The kernel a checked product takes (not the matvec, not MXFP4), and what it

@@ -201,3 +201,22 @@ def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
     lib.synchronize()
     assert np.all(np.abs(y.read(np.float32).reshape(m, n) - want) <= O.roundoff_bound(want, size, k, False))
 
+
+
+@pytest.mark.parametrize("fmt,m,n,k,kernel", [(P.Q8_0, 500, 2047, 256, 3), (P.Q6_K, 500, 2047, 256, 3), (P.Q4_K, 500, 2047, 256, 4),
+                                              (P.Q8_0, 300, 515, 512, 3), (P.Q4_K, 300, 515, 512, 3), (P.Q8_0, 300, 515, 1024, 5), (P.Q8_0, 1000, 1030, 768, 3),
+                                              (P.Q5_K, 300, 515, 512, 5), (P.Q6_K, 300, 515, 768, 5)])
+def test_odd_rows_of_a_short_k(lib, fmt, m, n, k, kernel):
+    """The fused tiles (3), the panel kernel (4) and the pass + GEMM (5) stand
+    side by side at short K, and an override reaches the one it names."""
+    from oco_amd import synth
+    say("odd rows, short k", fmt, m, n, k)
+    w = weights(fmt, n, k, 41)
+    x = synth.bf16_bits(synth.activations(42, m * k)).reshape(m, k)
+    half, mag = O.matmul_reference(fmt, w, x, n, k, half_operands=True)
+    p = lib.Matrix(k, n, m, 0, 1, 1, 0)
+    for values, want in (((), kernel), ((0,), 3), ((1,), 5)):
+        with lib.overridden(lib.Knob.MATMUL_VENDOR, values):
+            assert lib.matmul_route(fmt, p)[0] == want
+            got = product(lib, fmt, w, x, m, n, k, workspace=True)
+        assert np.all(np.abs(got - half) <= O.roundoff_bound(half, mag, k, False))
