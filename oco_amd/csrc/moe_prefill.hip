@@ -108,11 +108,11 @@ __device__ __forceinline__ void q4_static_for(F &&f) {
     }
 }
 
-// s_waitcnt vmcnt(N) (gfx9 encoding; expcnt and lgkmcnt left at their maxima).
+// s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding; expcnt left at its maximum).
 template <int N>
 __device__ __forceinline__ void q4_vm_wait() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
 }
 
 // Max over the 16 lanes of a DPP row (lanes 16 r .. 16 r + 15).
@@ -443,7 +443,9 @@ __global__ __launch_bounds__(64 * NW) void moe_q4k_kernel(KPRE_PARAMS, MatmulArg
     // wavefront, a finished unit's stores go out, and wc is marked in use
     // (the compiler's own wait for it then sits here, where it has landed).
     auto start = [&](int t, const Q4Set *wc) __attribute__((always_inline)) {
-        q4_vm_wait<LOADS>();                      // step t's loads (step t + 1's may be in flight)
+        // Step t's loads are here (step t + 1's may be in flight), and so are
+        // the last step's LDS reads: their stage is overwritten after the barrier.
+        q4_vm_wait<LOADS>();
         asm volatile("s_barrier" ::: "memory");  // every wavefront's LDS loads landed; stage (t + 2) % 3 is free
 #pragma unroll
         for (int i = 0; i < 5; i++) q4_touch(wc->c[i]);

@@ -35,8 +35,8 @@ struct PanelArgs {
     uint32_t y_bf16;
 };
 
-// s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima
-__device__ __forceinline__ void panel_vm_wait() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
+// s_waitcnt vmcnt(0) lgkmcnt(0), expcnt left at its maximum
+__device__ __forceinline__ void panel_wait() { __builtin_amdgcn_s_waitcnt(7 << 4); }
 
 template <int B, int E, typename F>
 __device__ __forceinline__ void panel_for(F &&f) {
@@ -94,8 +94,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void p
     };
     constexpr int ITEMS = NT + XL, RUNS = 6;  // spread over the first six of a step's eight runs
     auto step = [&](uint32_t u, const uint8_t *xs, U *w, uint8_t *xn, U *wn) __attribute__((always_inline)) {
-        panel_vm_wait();                          // this step's activations are in LDS, its weights here
-        asm volatile("s_barrier" ::: "memory");  // ... in every wavefront; the other buffer is free
+        // This step's activations are in LDS and its weights here, and the last
+        // step's LDS reads are done: their buffer is overwritten after the barrier.
+        panel_wait();
+        asm volatile("s_barrier" ::: "memory");
 #pragma unroll
         for (int t = 0; t < NT; t++) w[t].prep(q);
         panel_for<0, 8>([&](auto cc) __attribute__((always_inline)) {
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void p
         step(u, xs0, w0, xs1, w1);
         if (u + 1 < u1) step(u + 1, xs1, w1, xs0, w0);  // uniform
     }
-    panel_vm_wait();  // no load into LDS outlives the workgroup
+    panel_wait();  // no load into LDS outlives the workgroup
 
     // lane: activation row l % 16 of its tile, weight rows 4 (l / 16) .. + 4
     const bool quads = a.n % 4 == 0 && ((uintptr_t)(a.part ? (void *)a.part : a.y) & 15) == 0;
