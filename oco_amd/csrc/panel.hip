@@ -46,8 +46,11 @@ __device__ __forceinline__ void panel_for(F &&f) {
     }
 }
 
+// Registers for two workgroups on a CU where the LDS holds two (up to 64 rows):
+// Q4_K's 64 x 192 would take 264 and leave one, 512 rows of 12288 x 4096 97.6 us
+// against 78.6.
 template <int FMT, int MT, int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void panel_kernel(KPRE_PARAMS, PanelArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 8 ? 1 : 2))) void panel_kernel(KPRE_PARAMS, PanelArgs a) {
     KPRE_APPLY(a);
     using U = WeightUnit<FMT>;
     constexpr int BM = 16 * MT, XL = BM / 8;  // 16-byte activation loads per lane and step

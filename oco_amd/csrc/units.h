@@ -23,10 +23,7 @@ __device__ __forceinline__ f16x2 f16_pair(uint32_t bits) {
 __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
     asm("" : "+v"(a));
     asm("" : "+v"(b));
-    const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
-    uint32_t r;
-    __builtin_memcpy(&r, &h, 4);
-    return r;
+    return f16_bits(a, b);
 }
 // Four f16 of a * code - m from the bytes of one dword (a * code exact in f32).
 __device__ __forceinline__ void four_ub(uint32_t n, float a, float m, uint32_t &p01, uint32_t &p23) {
@@ -34,12 +31,6 @@ __device__ __forceinline__ void four_ub(uint32_t n, float a, float m, uint32_t &
     const float f2 = __builtin_fmaf(a, ub(n, 2), -m), f3 = __builtin_fmaf(a, ub(n, 3), -m);
     p01 = pk_f16(f0, f1);
     p23 = pk_f16(f2, f3);
-}
-__device__ __forceinline__ void q4_four_s(uint32_t n, float a, float m, uint32_t &p01, uint32_t &p23) {
-    const q4f32x2 c01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(n, 512.0f, false);
-    const q4f32x2 c23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(n, 512.0f, true);
-    p01 = pk_f16(__builtin_fmaf(a, c01[0], -m), __builtin_fmaf(a, c01[1], -m));
-    p23 = pk_f16(__builtin_fmaf(a, c23[0], -m), __builtin_fmaf(a, c23[1], -m));
 }
 
 // Buffer loads at any byte offset, zero past the resource's range.
@@ -108,7 +99,7 @@ struct WeightK4 {  // Q4_K, Q5_K: quarter q = sub-blocks 2q (runs 0-3) and 2q + 
                 n |= ((h[2 * (i & 1) + j] >> (2 * q + (i >= 4))) & 0x01010101u) << 4;
                 four_ub(n, a, m, out[2 * j], out[2 * j + 1]);
             } else {
-                q4_four_s(n, a, m, out[2 * j], out[2 * j + 1]);
+                q4_four(n, a, m, out[2 * j], out[2 * j + 1]);
             }
         }
     }
@@ -259,7 +250,7 @@ struct WeightQ4 {
                 __builtin_memcpy(&out[2 * j], &p01, 4);
                 __builtin_memcpy(&out[2 * j + 1], &p23, 4);
             } else {
-                q4_four_s(n, d[blk], m[blk], out[2 * j], out[2 * j + 1]);
+                q4_four(n, d[blk], m[blk], out[2 * j], out[2 * j + 1]);
             }
         }
     }
