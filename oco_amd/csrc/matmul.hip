@@ -977,24 +977,25 @@ static bool use_skinny(uint32_t format, const oco_matrix *p) {
 
 // Rows that are not whole quads over a short K: the fused tiles' one launch
 // against the panel kernel's two or three and the pass + GEMM's.  The fused
-// tiles' time is their K steps while they fill the chip once, the GEMM's grows
-// with the outputs.  (us; fused, then panel or GEMM; weights from HBM.)
-//   k = 256:  Q8_0 2047 at 1000 rows 8.4, panel 13.0; 8191 at 200 rows 8.9,
-//             panel 12.2, at 1000 rows 33.6, GEMM 46; Q6_K 38.5, 48.1
-//   k = 512:  Q8_0 2047 at 300 rows 11.3, GEMM 14.9; 4097 at 1000 rows 44, 31
-//   k = 1024: Q8_0 515 at 300 rows 18.6, GEMM 14.3; 2047 at 300 rows 19.0,
-//             17.5, at 1000 rows 20.9, 26.7; Q4_K 4097 at 300 rows 21.4, 24.8;
-//             Q6_K 26.0, 24.8
-// Q4 formats: the panel kernel, where it is chosen, is mostly the shorter
-// (8191 x 256 at 1000 rows 33.7, 27.7; 2047 x 256 9.1, 10.3).  Q5_K's fused
-// decode never is (2047 x 512 at 300 rows 47, GEMM 19).
+// tiles' time is their K steps while they fill the chip once, the others' grows
+// with the outputs.  (us; fused, then panel, then GEMM; weights from HBM.)
+//   k = 256:  Q8_0 2047 at 200 rows 7.2, 6.9, 10.5; 500 rows 7.5, 8.3, 13.9; 1000
+//             rows 8.7, 10.7, 18.3; 8191 at 200 rows 8.5, 10.2, 19.6; 500 rows
+//             17.0, 17.2, 28.5; Q6_K 8191 at 100 rows 8.7, 9.4, 17.8
+//   k = 512:  Q8_0 2047 at 300 rows 10.2, 9.0, 13.2; 1000 rows 12.3, 13.3, 20.5
+//   k = 1024: Q8_0 515 at 300 rows 16.9, 10.5, 11.9; 2047 at 1000 rows 19.5,
+//             17.7, 25.8; Q6_K 4097 at 300 rows 26.0, 18.8, 23.6
+// Q4 formats: the panel kernel is the shorter or within 8% (Q4_K 2047 x 256 at
+// 1000 rows 9.6, 10.3, 19.0).  Q5_K's fused decode never is (2047 x 512 at 300
+// rows 46, 9, 18).
 static bool use_short_rows(uint32_t format, const oco_matrix *p, bool panel) {
     const uint64_t mn = (uint64_t)p->m * p->n;
-    if (p->n % 4 == 0 || p->k > 1024 || mn > (p->k <= 256 ? 1u << 24 : 1u << 21) || (p->k > 512 && mn < 15u << 16)) return false;
+    if (p->n % 4 == 0 || p->k > 1024) return false;
+    if (panel) return (format == OCO_Q8_0 || format == OCO_Q6_K) && p->k <= 256 && mn >= 1u << 19 && mn <= 1u << 21;
+    if (mn > (p->k <= 256 ? 1u << 24 : 1u << 21) || (p->k > 512 && mn < 15u << 16)) return false;
     switch (format) {
-    case OCO_Q8_0: return p->k <= 256 || !panel;
-    case OCO_Q6_K: return p->k <= 256 || (p->k <= 512 && !panel);
-    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: return !panel;
+    case OCO_Q6_K: return p->k <= 512;
+    case OCO_Q8_0: case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: return true;
     }
     return false;
 }

@@ -17,8 +17,6 @@
 // MFMA and about 80 NT of decode (Q4_K), which do not overlap on one SIMD.
 #include "panel.h"
 
-#include <cmath>
-
 #include "units.h"
 
 namespace oco {
@@ -183,10 +181,12 @@ typedef void (*PanelFn)(u32x4, u32x4, u32x4, u32x2, PanelArgs);
 // The tiles in use: (16-row activation tiles, 16-row weight tiles per
 // wavefront).  Wider ones at eight activation tiles (128 x 128, 128 x 192)
 // leave one wavefront per SIMD with nothing to cover its waits and measured
-// slower than 64 x 192 at every size.
+// slower than 64 x 192 at every size; 128 x 64 pays for the largest decode
+// only (Q6_K 12288 x 4096 at 128 rows 48.0 us, 64 x 64 55.8).
 template <int FMT>
 static PanelFn panel_pick(int mt, int nt) {
-    if (mt == 8) return panel_kernel<FMT, 8, 1>;
+    if constexpr (FMT == OCO_Q6_K)
+        if (mt == 8) return panel_kernel<FMT, 8, 1>;
     if constexpr (FMT == OCO_Q4_K || FMT == OCO_Q4_0 || FMT == OCO_Q4_1) {
         if (nt == 3) return panel_kernel<FMT, 4, 3>;
         if (nt == 2) return panel_kernel<FMT, 4, 2>;
@@ -194,74 +194,86 @@ static PanelFn panel_pick(int mt, int nt) {
     return mt == 4 ? panel_kernel<FMT, 4, 1> : panel_kernel<FMT, 2, 1>;
 }
 
-// Measured per 256 columns (Q4_K, us): a workgroup alone on its CU, and per
-// workgroup with the CU full (weights in the Infinity Cache; streamed from
-// HBM the products of 256 rows and more take about 10% longer on both paths).  Other formats add their decode per weight tile.
+// What a tile takes, in us: once per call (launches included), once more per
+// workgroup that a CU runs, and per 256 columns for a workgroup alone on its
+// CU and for two that share it (zero: not built for the format).  A CU that
+// runs three takes a pair's time and one alone's, and so on: 64 x 192 of Q4_K
+// steps at 2.8, 4.2-4.6, 6.2, 7.8 for one to four.  Fitted, with the estimates
+// below, to 2900 timings of 83 matrices (256 to 151936 rows, K 256 to 28672) at
+// 32 to 1000 rows, with weights streamed from HBM, in long runs; they miss them by
+// 8% (root mean square).
 struct PanelTile {
     int mt, nt;
-    double alone, full;
+    double start, more;
+    struct {
+        double alone, pair;
+    } step[4];  // by panel_class
 };
-static const PanelTile PANEL_TILES[] = {{4, 3, 3.34, 2.37}, {4, 2, 2.4, 1.8}, {8, 1, 2.1, 2.1}, {4, 1, 1.43, 0.91}, {2, 1, 0.98, 0.55}};
+static const PanelTile PANEL_TILES[] = {{4, 3, 8.2, 0.0, {{2.05, 3.55}, {3.1, 4.4}, {}, {}}},
+                                        {4, 2, 6.7, 0.4, {{1.55, 2.55}, {2.1, 3.2}, {}, {}}},
+                                        {8, 1, 4.5, 2.5, {{}, {}, {}, {2.4, 4.7}}},
+                                        {4, 1, 5.0, 0.7, {{1.0, 1.48}, {1.37, 2.1}, {1.53, 2.2}, {1.84, 2.85}}},
+                                        {2, 1, 5.1, 0.1, {{0.76, 1.07}, {1.13, 1.43}, {1.2, 1.82}, {1.68, 2.58}}}};
 
-// us per 256 columns and weight tile that a format's decode adds; below zero:
-// not decoded here.
-static double panel_decode(uint32_t format) {
+// Formats of about the same decode; below zero: not decoded here.
+static int panel_class(uint32_t format) {
     switch (format) {
-    case OCO_Q4_0: case OCO_Q4_1: case OCO_Q4_K: return 0;
-    case OCO_Q8_0: case OCO_Q5_K: return 0.33;
-    case OCO_Q6_K: return 0.55;
+    case OCO_Q4_K: return 0;
+    case OCO_Q4_0: case OCO_Q4_1: return 1;
+    case OCO_Q8_0: case OCO_Q5_K: return 2;
+    case OCO_Q6_K: return 3;
     }
     return -1;
 }
 
+static uint64_t panel_workgroups(int mt, int nt, uint64_t s, uint32_t m, uint32_t n) {
+    return (uint64_t)((n + 64 * nt - 1) / (64 * nt)) * ((m + 16 * mt - 1) / (16 * mt)) * s;
+}
+
 bool panel_fits(uint32_t format, const PanelPlan &pl, uint32_t m, uint32_t n, uint32_t k) {
-    const double decode = panel_decode(format);
-    if (decode < 0 || k == 0 || k % 256 || m == 0 || n == 0 || m > 0x3fffffffu || n > 0x3fffffffu) return false;
+    const int cls = panel_class(format);
+    if (cls < 0 || k == 0 || k % 256 || m == 0 || n == 0 || m > 0x3fffffffu || n > 0x3fffffffu) return false;
     bool built = false;
-    for (const PanelTile &t : PANEL_TILES) built = built || (t.mt == pl.mt && t.nt == pl.nt && (t.nt == 1 || decode == 0));
+    for (const PanelTile &t : PANEL_TILES) built = built || (t.mt == pl.mt && t.nt == pl.nt && t.step[cls].alone > 0);
     if (!built || 64ull * pl.nt * oco_row_bytes(format, k) >= UNIT_OFF) return false;
     const uint64_t s = pl.splits;
     if (s == 0 || s > k / 256 || (s > 1 && s * m * 2 > k)) return false;  // the parts lie where the pass's f16 weights would
-    return (uint64_t)((n + 64 * pl.nt - 1) / (64 * pl.nt)) * ((m + 16 * pl.mt - 1) / (16 * pl.mt)) * s < 0x80000000ull;
+    return panel_workgroups(pl.mt, pl.nt, s, m, n) < 0x80000000ull;
 }
 
 // The tile and the K parts by estimated time, and whether that beats the
-// dequantize pass + GEMM + epilogue.  Both estimates are fits to
-// measurements (Q4_K 12288 x 4096, bf16 out, us, pass and GEMM against this):
-// 32 rows 50.0, 18.2; 64 rows 52.6, 23.7; 128 rows 63.6, 34.7; 256 rows 72.3,
-// 54.2; 512 rows 97, 81.  Q6_K 4096 x 12288: 64 rows 64.7, 33.2; 200 rows
-// 81.1, 70.5; 512 rows 117, 132.  Q8_0 4096 x 4096: 64 rows 22.9, 14.9; 256
-// rows 30.8, 28.7; 512 rows 39.1, 44.  Past a few hundred rows the decode is
-// repeated too often (once per 64 or 128 rows) against one pass for all.
+// dequantize pass + GEMM + epilogue, whose time depends on the kernel the
+// library takes and is not monotone in the rows (Q4_K 12288 x 4096 at 352,
+// 416 and 480 rows: 74, 100 and 81 us): its estimate lies low, 0.75 to 1.13 times
+// the measured (5th and 95th percentile), so that the panel kernel is taken
+// where its lead holds, and a few percent are asked for on top.  Of 960 streamed
+// products three are more than 2% slower here than on the GEMM, at most 6%, and the
+// choice is 1.02 times the fastest of all on average.  Q4_K 12288 x 4096,
+// bf16 out, us, pass and GEMM against this: 32 rows 51, 19; 64 rows 50, 25; 128
+// rows 66, 35; 256 rows 72, 51; 512 rows 85, 81; 14336 x 4096 at 448 rows 88
+// against 94 to 106 on the tiles here, which are not taken.
 PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
     PanelPlan best = {};
-    const double decode = panel_decode(format);
+    const int cls = panel_class(format);
     if (!panel_fits(format, {2, 1, 1}, m, n, k)) return best;
-    const double row_bytes = (double)oco_row_bytes(format, k), passes = 5.1e6;  // bytes per us of the passes over memory
-    const double mn = (double)m * n, gemm = std::max(k / 512.0, 1.6 * n * k / passes + mn * k / 0.65e9),
-                 vendor = 8 + (n * (2.0 * k + row_bytes) + 4.0 * m * k + 10 * mn) / passes + gemm;
-    const uint32_t units = k / 256;
-    // Margins for what the fits miss, the larger decodes and many rows most:
-    // with weights streamed from HBM, 384 rows of Q4_K 12288 x 4096 took 79 us
-    // here against 77, 512 rows 83 against 87.
-    double least = (m > 512 || decode > 0 ? 0.8 : m > 256 ? 0.82 : 0.92) * vendor;
-    for (const PanelTile &t : PANEL_TILES) {
+    const double mn = 1e-6 * m * n, mk = 1e-6 * m * k, nk = 1e-6 * n * k;
+    // us per 10^6 weights of the pass
+    const double pass = format == OCO_Q5_K ? 1.75 : cls == 1 ? 0.98 : 0.72;
+    const double gemm = 9 + 1.25e-3 * k + pass * nk + (2.6 + 2.6 * std::min(k, 8192u) / 4096) * mn + 2 * mk;
+    const double stream = 1e-6 * n * oco_row_bytes(format, k) / 5.1;  // the weights at the rate of a copy
+    double least = 0.96 * gemm;
+    for (const PanelTile &t : PANEL_TILES)
         for (uint32_t s = 1; s <= 8; s *= 2) {
             if (!panel_fits(format, {t.mt, t.nt, s}, m, n, k)) break;
-            const double wgs = std::ceil(n / (64.0 * t.nt)) * std::ceil(m / (16.0 * t.mt)) * s;
-            // Past 256 rows: by the fullest CU while two workgroups share it, and
-            // only the widest tile for more (it decodes least per product).
-            double load = wgs / 256;
-            if (m > 256 && load <= 2) load = std::ceil(load);
-            if (m > 256 && load > 2 && t.nt < 3) continue;
-            const double step = std::max(t.alone + t.nt * decode, load * (t.full + t.nt * decode));
-            const double us = 6 + std::ceil((double)units / s) * step + (s > 1 ? 2.5 + 8.0 * s * mn / passes : 0);
+            const uint64_t load = (panel_workgroups(t.mt, t.nt, s, m, n) + 255) / 256;  // on the fullest CU
+            const double step = (load % 2) * t.step[cls].alone + (load / 2) * t.step[cls].pair;
+            const double us = t.start + t.more * load + std::max((k / 256 + s - 1) / s * step, stream) + 0.95 * mk + 0.9 * mn +
+                              (s > 1 ? 1.2 + 0.32 * s + 1.4 * s * mn : 0);  // the parts and their sum
             if (us < least) {
                 least = us;
                 best = {t.mt, t.nt, s};
             }
         }
-    }
     return best;
 }
 

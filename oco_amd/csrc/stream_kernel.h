@@ -230,7 +230,8 @@ __global__ __launch_bounds__(256) void stream_kernel(const uint8_t *w_, const vo
     float xv[NPL][32], sv[NPL][NS];
     // The first 1024 float4 of x are requested before the weights: they come
     // from L2 and arrive while the weights are still in flight (loads return
-    // in issue order).  A fused norm reads x itself first, so it does not.
+    // in issue order).  A fused norm (block_inv_rms below) reads x after the
+    // weights have been requested, so its sum follows their arrival.
     const XT *xr = reinterpret_cast<const XT *>(a.x) + (uint64_t)input * p.k;
     float xpre[4][4];
     if constexpr (XS == XS_STAGED) {

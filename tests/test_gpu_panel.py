@@ -34,7 +34,7 @@ def test_prompt_chunk(lib, fmt, m, n, k):
 
 Q4 = (P.Q4_0, P.Q4_1, P.Q4_K)  # the formats of the wider tiles
 TILES = [(fmt, mt, nt) for fmt in (P.Q8_0, P.Q4_K, P.Q5_K, P.Q6_K, P.Q4_0, P.Q4_1)
-         for mt, nt in [(2, 1), (4, 1), (8, 1), (4, 2), (4, 3)] if nt == 1 or fmt in Q4]
+         for mt, nt in [(2, 1), (4, 1), (8, 1), (4, 2), (4, 3)] if (mt < 8 or fmt == P.Q6_K) and (nt == 1 or fmt in Q4)]
 
 
 @pytest.mark.parametrize("fmt,mt,nt", TILES)
@@ -67,7 +67,22 @@ def test_every_tile(lib, fmt, mt, nt):
         assert np.all(np.abs(got - want) <= bound), (parts, m, n, k, np.abs(got - want).max())
 
 
-@pytest.mark.parametrize("fmt,values,m,k", [(P.Q4_K, (2, 3, 1, 1), 64, 512), (P.Q8_0, (2, 4, 2, 1), 64, 512), (P.Q4_K, (2, 4, 1, 3), 40, 512),
+@pytest.mark.parametrize("fmt,n,k,choices", [
+    (P.Q4_K, 12288, 4096, {32: (2, 1, 2), 128: (4, 1, 1), 256: (4, 3, 1), 320: (4, 2, 1), 512: (4, 3, 1), 640: None, 1024: None}),
+    (P.Q4_K, 14336, 4096, {32: (2, 1, 2), 256: (4, 2, 1), 384: (4, 3, 1), 448: None, 512: None, 640: None}),
+    (P.Q8_0, 4096, 4096, {64: (4, 1, 4), 256: (4, 1, 2), 512: None}), (P.Q6_K, 12288, 4096, {64: (4, 1, 4), 128: (8, 1, 1), 512: None}),
+    (P.Q5_K, 4096, 4096, {64: (4, 1, 4), 448: (4, 1, 1), 1024: None}),
+    (P.Q4_0, 12288, 4096, {64: (4, 2, 4), 128: (4, 3, 4), 512: (4, 3, 1), 640: None})])
+def test_choice(lib, fmt, n, k, choices):
+    """Tile and K parts, or the pass + GEMM (None), at row counts whose times
+    on both are known (64 x 192 of 14336 x 4096 needs a third workgroup on some CUs
+    from 448 rows on)."""
+    for m, tile in choices.items():
+        kernel, *got = lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 0))
+        assert (kernel, *got) == ((lib.MatmulKernel.PANEL, *tile) if tile else (lib.MatmulKernel.GEMM, 0, 0, 0)), m
+
+
+@pytest.mark.parametrize("fmt,values,m,k", [(P.Q4_K, (2, 3, 1, 1), 64, 512), (P.Q8_0, (2, 4, 2, 1), 64, 512), (P.Q4_K, (2, 8, 1, 1), 64, 512), (P.Q4_K, (2, 4, 1, 3), 40, 512),
                                             (P.Q4_K, (2, 4, 1, 2), 200, 512), (P.Q4_K, (2, 4, 1, 0), 64, 512), (P.Q4_K, (2,), 64, 512),
                                             (P.Q8_0, (2, 4, 1, 1), 64, 288), (1, (2, 4, 1, 1), 64, 512)])
 def test_a_pinned_tile_that_cannot_run_is_refused(lib, fmt, values, m, k):
@@ -202,10 +217,9 @@ def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
     assert np.all(np.abs(y.read(np.float32).reshape(m, n) - want) <= O.roundoff_bound(want, size, k, False))
 
 
-
-@pytest.mark.parametrize("fmt,m,n,k,kernel", [(P.Q8_0, 500, 2047, 256, 3), (P.Q6_K, 500, 2047, 256, 3), (P.Q4_K, 500, 2047, 256, 4),
-                                              (P.Q8_0, 300, 515, 512, 3), (P.Q4_K, 300, 515, 512, 3), (P.Q8_0, 300, 515, 1024, 5), (P.Q8_0, 1000, 1030, 768, 3),
-                                              (P.Q5_K, 300, 515, 512, 5), (P.Q6_K, 300, 515, 768, 5)])
+@pytest.mark.parametrize("fmt,m,n,k,kernel", [(P.Q8_0, 500, 2047, 256, 3), (P.Q6_K, 500, 2047, 256, 3), (P.Q8_0, 200, 2047, 256, 4), (P.Q8_0, 400, 8191, 256, 4),
+                                              (P.Q4_K, 500, 2047, 256, 4), (P.Q8_0, 300, 515, 480, 3), (P.Q8_0, 300, 515, 512, 4), (P.Q8_0, 300, 515, 992, 5),
+                                              (P.Q8_0, 1000, 1030, 736, 3), (P.Q5_K, 300, 515, 512, 4), (P.Q6_K, 700, 4097, 1024, 5)])
 def test_odd_rows_of_a_short_k(lib, fmt, m, n, k, kernel):
     """The fused tiles (3), the panel kernel (4) and the pass + GEMM (5) stand
     side by side at short K, and an override reaches the one it names."""
