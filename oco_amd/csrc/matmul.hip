@@ -730,19 +730,27 @@ static const BlasPlan &blas_plan(uint32_t m, uint32_t n, uint32_t k) {
         hipblasLtMatrixLayoutCreate(&pl.b, HIP_R_16F, k, m, k) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&pl.d, HIP_R_32F, n, m, n) != HIPBLAS_STATUS_SUCCESS)
         return pl;
+    // The library's order without a limit on the workspace, and of that the
+    // first within BLAS_WS_MAX.  Under a limit it cuts the K parts of the
+    // algorithms that exceed it: to a part of their workspace, which the product
+    // then refuses (status 6: 416 rows of 4096 x 12288), or to one part (1999 rows
+    // of it 204 us, here 127).  One that needs no workspace is always offered.
     hipblasLtMatmulPreference_t pref = nullptr;
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return pl;
-    const uint64_t wsmax = BLAS_WS_MAX;
-    hipblasLtMatmulHeuristicResult_t res;
-    int count = 0;
-    if (hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsmax, sizeof(wsmax)) ==
-            HIPBLAS_STATUS_SUCCESS &&
-        hipblasLtMatmulAlgoGetHeuristic(h, pl.desc, pl.a, pl.b, pl.d, pl.d, pref, 1, &res, &count) ==
-            HIPBLAS_STATUS_SUCCESS &&
-        count > 0 && res.state == HIPBLAS_STATUS_SUCCESS && res.workspaceSize <= BLAS_WS_MAX) {
-        pl.algo = res.algo;
-        pl.ws = res.workspaceSize;
-        pl.ok = true;
+    for (uint64_t wsmax : {uint64_t(1) << 40, uint64_t(0)}) {
+        hipblasLtMatmulHeuristicResult_t res[16];
+        int count = 0;
+        if (hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsmax, sizeof(wsmax)) !=
+                HIPBLAS_STATUS_SUCCESS ||
+            hipblasLtMatmulAlgoGetHeuristic(h, pl.desc, pl.a, pl.b, pl.d, pl.d, pref, 16, res, &count) != HIPBLAS_STATUS_SUCCESS)
+            continue;
+        for (int i = 0; i < count && !pl.ok; i++)
+            if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= BLAS_WS_MAX) {
+                pl.algo = res[i].algo;
+                pl.ws = res[i].workspaceSize;
+                pl.ok = true;
+            }
+        if (pl.ok) break;
     }
     hipblasLtMatmulPreferenceDestroy(pref);
     return pl;

@@ -15,7 +15,7 @@ import pytest
 
 import oracle as O
 import packers as P
-from _util import Guarded, rel_l2, say
+from _util import SENTINEL, Guarded, rel_l2, say
 
 pytestmark = pytest.mark.gpu
 
@@ -351,6 +351,40 @@ def test_matmul_vendor_in_graph(lib):
         assert np.array_equal(y.download(np.uint16, m * n), want)
         lib.matmul(fmt, w, x, eager, p, y_dtype=lib.DType.BF16)  # eager work between replays
         lib.synchronize()
+
+
+@pytest.mark.parametrize("m,n,k", [(416, 4096, 12288), (700, 2560, 9728), (832, 4098, 11008), (1536, 2560, 9728)])
+def test_matmul_gemm_over_a_long_k(lib, m, n, k):
+    """Shapes whose first choice in the GEMM library needs more workspace than
+    is given: within the bounds on a sample of rows, the workspace used as
+    reported, and three graph replays equal to the eager result bit for bit."""
+    from oco_amd import synth
+    say("matmul long k", m, n, k)
+    w = synth.weights(P.Q8_0, n, k, seed=45)
+    x = synth.bf16_bits(synth.activations(46, m * k)).reshape(m, k)
+    wb, xb, p = lib.DeviceBuffer.from_array(w), lib.DeviceBuffer.from_array(x), lib.Matrix(k, n, m, 0, 1, 1, 0)
+    with lib.overridden(lib.Knob.MATMUL_VENDOR, (1,)):
+        need = lib.matmul_workspace(P.Q8_0, p)
+        ws = lib.DeviceBuffer(need + 256)
+        ws.fill32(SENTINEL)
+        run_into = lambda out, s=None: lib.matmul(P.Q8_0, wb, xb, out, p, stream=s, workspace=ws, workspace_bytes=need)  # noqa: E731
+        eager, y, s = Guarded(lib, m * n * 4), lib.DeviceBuffer(m * n * 4), lib.Stream()
+        run_into(eager.ptr)
+        lib.synchronize()
+        want = eager.read(np.float32)
+        g = lib.Graph(s, lambda: run_into(y, s))
+        for _ in range(3):
+            y.fill32(0)
+            lib.synchronize()
+            g.launch()
+            s.sync()
+            np.testing.assert_array_equal(y.download(np.float32), want)
+            run_into(eager.ptr)
+            lib.synchronize()
+    assert np.all(ws.download(np.uint32, 64, need) == SENTINEL)  # nothing past the workspace
+    got, rows = want.reshape(m, n), np.r_[0, 1, m // 2, m - 1]
+    half, mag = O.matmul_reference(P.Q8_0, w, x[rows], n, k, half_operands=True)
+    assert np.all(np.abs(got[rows] - half) <= O.roundoff_bound(half, mag, k, False))
 
 
 def test_matmul_f16_input_unaligned(lib):
