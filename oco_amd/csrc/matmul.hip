@@ -980,7 +980,7 @@ static bool matmul_override() {
 }
 
 static bool use_skinny(uint32_t format, const oco_matrix *p) {
-    return p->m < 32 && !matmul_override() && skinny_fits(format, p->m, p->n, p->k);
+    return !matmul_override() && skinny_fits(format, p->m, p->n, p->k);
 }
 
 // Rows that are not whole quads over a short K: the fused tiles' one launch

@@ -1,4 +1,4 @@
-// Y[m, n] = X[m, k] W[n, k]^T for a few activation rows (m <= 32): decode
+// Y[m, n] = X[m, k] W[n, k]^T for a few activation rows (m <= SKINNY_ROWS): decode
 // batches, draft verification, short prompts.  Replaces the small-m plans of
 // DenseMatrix::apply (src/weights/compute/matrix.rs:130-379) on the same
 // operands as the larger tiles here: half(w) and half(x), fp32 accumulation.
