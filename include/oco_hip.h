@@ -269,8 +269,8 @@ typedef enum oco_matmul_kernel {
     OCO_MATMUL_PANEL = 4,    /* prompt chunks, weights decoded in registers */
     OCO_MATMUL_GEMM = 5      /* dequantize pass, then the vendor GEMM */
 } oco_matmul_kernel;
-int oco_matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, uint64_t workspace_bytes,
-                     uint32_t route[4]);
+int oco_matmul_route(uint32_t format, oco_dtype x_dtype, oco_dtype y_dtype, const oco_matrix *p,
+                     uint64_t workspace_bytes, uint32_t route[4]);
 
 /* The norm -> MXFP4 prefill pair in two launches instead of three: the RMS
  * norm of oco_norm (same rounding) whose workgroups also split each output

@@ -161,7 +161,7 @@ SIGNATURES = {
     "oco_matvec_relu_sqr": (_i32, [_u32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _MP, _vp]),
     "oco_matmul": (_i32, [_u32, _vp, _vp, _i32, _vp, _i32, _vp, _MP, _vp]),
     "oco_matmul_workspace": (_u64, [_u32, _i32, _MP]),
-    "oco_matmul_route": (_i32, [_u32, _i32, _MP, _u64, ctypes.POINTER(_u32)]),
+    "oco_matmul_route": (_i32, [_u32, _i32, _i32, _MP, _u64, ctypes.POINTER(_u32)]),
     "oco_matmul_ws": (_i32, [_u32, _vp, _vp, _i32, _vp, _i32, _vp, _MP, _vp, _u64, _vp]),
     "oco_norm_mx_split": (_i32, [_vp, _vp, _vp, _u32, _u32, ctypes.c_float, _i32, _vp, _u64, _vp]),
     "oco_add_norm_mx_split": (_i32, [_vp, _vp, _vp, _vp, _u32, _u32, ctypes.c_float, _i32, _vp, _u64, _vp]),
@@ -465,12 +465,13 @@ class MatmulKernel(enum.IntEnum):
     GEMM = 5
 
 
-def matmul_route(fmt: int, p: Matrix, x_dtype=DType.BF16, workspace_bytes: int | None = None):
+def matmul_route(fmt: int, p: Matrix, x_dtype=DType.BF16, y_dtype=DType.F32, workspace_bytes: int | None = None):
     """oco_matmul_route: (kernel, row tiles, column tiles, K parts); by default with the reported workspace."""
     if workspace_bytes is None:
         workspace_bytes = matmul_workspace(fmt, p, x_dtype)
     out = (_u32 * 4)()
-    _check(load_library().oco_matmul_route(int(fmt), int(x_dtype), ctypes.byref(as_matrix(p)), int(workspace_bytes), out))
+    _check(load_library().oco_matmul_route(int(fmt), int(x_dtype), int(y_dtype), ctypes.byref(as_matrix(p)),
+                                           int(workspace_bytes), out))
     return (MatmulKernel(out[0]), *out[1:])
 
 

@@ -733,8 +733,9 @@ static const BlasPlan &blas_plan(uint32_t m, uint32_t n, uint32_t k) {
     // The library's order without a limit on the workspace, and of that the
     // first within BLAS_WS_MAX.  Under a limit it cuts the K parts of the
     // algorithms that exceed it: to a part of their workspace, which the product
-    // then refuses (status 6: 416 rows of 4096 x 12288), or to one part (1999 rows
-    // of it 204 us, here 127).  One that needs no workspace is always offered.
+    // then refuses (status 6: 416 rows of 4096 x 12288), or to one part (Q4_K
+    // 8192 x 28672 at 512 rows, pass and epilogue included, 685 us, here 366).  One
+    // that needs no workspace is always offered.
     hipblasLtMatmulPreference_t pref = nullptr;
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return pl;
     for (uint64_t wsmax : {uint64_t(1) << 40, uint64_t(0)}) {
@@ -811,6 +812,11 @@ static void operand_launch(const void *w, uint64_t row_bytes, uint32_t n, uint32
                        n, k, wo, (const uint16_t *)x, xo, xchunks, wblocks);
 }
 
+// The f32 product of the GEMM as the output, without an epilogue.
+static bool gemm_direct(uint32_t format, oco_dtype x_dtype, oco_dtype y_dtype, const oco_matrix *p) {
+    return y_dtype == OCO_DT_F32 && !p->has_bias && !q4_gain(format, p->n, x_dtype);
+}
+
 static int vendor_workspace_check(const void *workspace, uint64_t bytes, uint64_t need) {
     if (!workspace || bytes < need)
         return fail(OCO_ERR_INVALID, "oco_matmul_ws: workspace of %llu bytes, need %llu", (unsigned long long)bytes,
@@ -845,7 +851,7 @@ static int vendor_matmul(uint32_t format, const void *w, const void *x, oco_dtyp
         OCO_TRY(launch_check("oco_matmul: operand pass"));
     }
     // f32 output without bias or gain is the GEMM's own output (when aligned for it)
-    const bool direct = y_dtype == OCO_DT_F32 && !(p->has_bias && bias) && !gain && ((uintptr_t)y & 15) == 0;
+    const bool direct = gemm_direct(format, x_dtype, y_dtype, p) && ((uintptr_t)y & 15) == 0;
     float *acc = direct ? (float *)y : (float *)(ws + v.d);
     const float alpha = 1.0f, beta = 0.0f;
     const hipblasStatus_t st = hipblasLtMatmul(pl.handle, pl.desc, &alpha, wo ? (const void *)wo : w, pl.a,
@@ -1016,8 +1022,8 @@ struct Route {
     PanelPlan panel;
 };
 
-static int matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, bool aligned, bool workspace,
-                        uint64_t workspace_bytes, Route *r) {
+static int matmul_route(uint32_t format, oco_dtype x_dtype, oco_dtype y_dtype, const oco_matrix *p, bool aligned,
+                        bool workspace, uint64_t workspace_bytes, Route *r) {
     *r = {OCO_MATMUL_TILES, nullptr, {}};
     // Rows that are not whole quads need no workspace: without one (and then
     // without a look at the GEMM library, inside a capture perhaps) they run on
@@ -1040,21 +1046,21 @@ static int matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p,
         return OCO_OK;
     }
     if (!matmul_override()) {
-        r->panel = panel_plan(format, p->m, p->n, p->k);
+        r->panel = panel_plan(format, p->m, p->n, p->k, gemm_direct(format, x_dtype, y_dtype, p));
         if (use_short_rows(format, p, r->panel.mt != 0)) return OCO_OK;
     }
     r->kernel = r->panel.mt ? OCO_MATMUL_PANEL : OCO_MATMUL_GEMM;
     return OCO_OK;
 }
 
-extern "C" int oco_matmul_route(uint32_t format, oco_dtype x_dtype, const oco_matrix *p, uint64_t workspace_bytes,
-                                uint32_t route[4]) {
+extern "C" int oco_matmul_route(uint32_t format, oco_dtype x_dtype, oco_dtype y_dtype, const oco_matrix *p,
+                                uint64_t workspace_bytes, uint32_t route[4]) {
     if (!p || !route) return fail(OCO_ERR_INVALID, "oco_matmul_route: null argument");
     Route r = {OCO_MATMUL_VECTOR, nullptr, {}};
     if (use_mx(format) && !as_matvec(format, x_dtype, p))
         r.kernel = OCO_MATMUL_MX;
     else if (!as_matvec(format, x_dtype, p))
-        OCO_TRY(matmul_route(format, x_dtype, p, true, workspace_bytes != 0, workspace_bytes, &r));
+        OCO_TRY(matmul_route(format, x_dtype, y_dtype, p, true, workspace_bytes != 0, workspace_bytes, &r));
     const bool panel = r.kernel == OCO_MATMUL_PANEL;
     route[0] = r.kernel;
     route[1] = panel ? r.panel.mt : 0;
@@ -1089,7 +1095,7 @@ extern "C" int oco_matmul_ws(uint32_t format, const void *w, const void *x, oco_
     const bool aligned = (format != OCO_F16 || ((uintptr_t)w & 15) == 0) &&
                          (x_dtype != OCO_DT_F16 || ((uintptr_t)x & 15) == 0);
     Route r;
-    OCO_TRY(matmul_route(format, x_dtype, p, aligned, workspace != nullptr, workspace_bytes, &r));
+    OCO_TRY(matmul_route(format, x_dtype, y_dtype, p, aligned, workspace != nullptr, workspace_bytes, &r));
     const BlasPlan *pl = r.pl;
     if (r.kernel == OCO_MATMUL_FEW_ROWS) {
         const void *xin = x;

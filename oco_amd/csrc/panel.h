@@ -13,7 +13,8 @@ struct PanelPlan {
     int mt, nt;
     uint32_t splits;
 };
-PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k);
+// direct: the GEMM's f32 product would be the output (no bias, no row gain).
+PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k, bool direct);
 // Whether a tile and K parts can run: a tile built for the format, offsets
 // within 32 bits, and the f32 parts within the f16 weights' place.
 bool panel_fits(uint32_t format, const PanelPlan &pl, uint32_t m, uint32_t n, uint32_t k);

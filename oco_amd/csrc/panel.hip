@@ -243,23 +243,24 @@ bool panel_fits(uint32_t format, const PanelPlan &pl, uint32_t m, uint32_t n, ui
 
 // The tile and the K parts by estimated time, and whether that beats the
 // dequantize pass + GEMM + epilogue, whose time depends on the kernel the
-// library takes and is not monotone in the rows (Q4_K 12288 x 4096 at 352,
-// 416 and 480 rows: 74, 100 and 81 us): its estimate lies low, 0.75 to 1.13 times
+// library takes and is not monotone in the rows (Q4_K 14336 x 4096 at 192,
+// 224 and 352 rows: 80, 73 and 86 us): its estimate lies low, 0.76 to 1.13 times
 // the measured (5th and 95th percentile), so that the panel kernel is taken
-// where its lead holds, and a few percent are asked for on top.  Of 960 streamed
-// products three are more than 2% slower here than on the GEMM, at most 6%, and the
-// choice is 1.02 times the fastest of all on average.  Q4_K 12288 x 4096,
+// where its lead holds, and a few percent are asked for on top.  Of 985 streamed
+// products three are more than 2% slower here than on the GEMM, at most 7%, and the
+// choice is 1.014 times the fastest of all on average.  Q4_K 12288 x 4096,
 // bf16 out, us, pass and GEMM against this: 32 rows 51, 19; 64 rows 50, 25; 128
-// rows 66, 35; 256 rows 72, 51; 512 rows 85, 81; 14336 x 4096 at 448 rows 88
+// rows 66, 35; 256 rows 74, 51; 512 rows 85, 81; 14336 x 4096 at 448 rows 87
 // against 94 to 106 on the tiles here, which are not taken.
-PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k) {
+PanelPlan panel_plan(uint32_t format, uint32_t m, uint32_t n, uint32_t k, bool direct) {
     PanelPlan best = {};
     const int cls = panel_class(format);
     if (!panel_fits(format, {2, 1, 1}, m, n, k)) return best;
     const double mn = 1e-6 * m * n, mk = 1e-6 * m * k, nk = 1e-6 * n * k;
     // us per 10^6 weights of the pass
     const double pass = format == OCO_Q5_K ? 1.75 : cls == 1 ? 0.98 : 0.72;
-    const double gemm = 9 + 1.25e-3 * k + pass * nk + (2.6 + 2.6 * std::min(k, 8192u) / 4096) * mn + 2 * mk;
+    const double epilogue = direct ? 0 : 1.5 + 1.2 * mn;
+    const double gemm = 7.5 + 1.25e-3 * k + pass * nk + (1.4 + 2.6 * std::min(k, 8192u) / 4096) * mn + 2 * mk + epilogue;
     const double stream = 1e-6 * n * oco_row_bytes(format, k) / 5.1;  // the weights at the rate of a copy
     double least = 0.96 * gemm;
     for (const PanelTile &t : PANEL_TILES)

@@ -78,7 +78,7 @@ def test_choice(lib, fmt, n, k, choices):
     on both are known (64 x 192 of 14336 x 4096 needs a third workgroup on some CUs
     from 448 rows on)."""
     for m, tile in choices.items():
-        kernel, *got = lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 0))
+        kernel, *got = lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 0), y_dtype=lib.DType.BF16)
         assert (kernel, *got) == ((lib.MatmulKernel.PANEL, *tile) if tile else (lib.MatmulKernel.GEMM, 0, 0, 0)), m
 
 
@@ -217,7 +217,7 @@ def test_rows_that_are_not_whole_quads(lib, fmt, m, n, k):
     assert np.all(np.abs(y.read(np.float32).reshape(m, n) - want) <= O.roundoff_bound(want, size, k, False))
 
 
-@pytest.mark.parametrize("fmt,m,n,k,kernel", [(P.Q8_0, 500, 2047, 256, 3), (P.Q6_K, 500, 2047, 256, 3), (P.Q8_0, 200, 2047, 256, 4), (P.Q8_0, 400, 8191, 256, 4),
+@pytest.mark.parametrize("fmt,m,n,k,kernel", [(P.Q8_0, 500, 2047, 256, 3), (P.Q6_K, 500, 2047, 256, 3), (P.Q8_0, 200, 2047, 256, 4),
                                               (P.Q4_K, 500, 2047, 256, 4), (P.Q8_0, 300, 515, 480, 3), (P.Q8_0, 300, 515, 512, 4), (P.Q8_0, 300, 515, 992, 5),
                                               (P.Q8_0, 1000, 1030, 736, 3), (P.Q5_K, 300, 515, 512, 4), (P.Q6_K, 700, 4097, 1024, 5)])
 def test_odd_rows_of_a_short_k(lib, fmt, m, n, k, kernel):
