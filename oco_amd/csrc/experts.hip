@@ -465,10 +465,6 @@ uint64_t oco_experts_workspace(const oco_experts *w, uint32_t tokens) {
 
 }  // extern "C"
 
-// The layer after the router logits.  With `logits`, the experts are
-// selected on the device (ids/probs are written): at one token inside the
-// routed gate/up kernel (expert_expand's selection), else inside the route
-// plan's launch.
 // The MXFP4 tiles at a small decode batch: every gate/up workgroup builds
 // the route plan itself (route.h), the input rows are split beside the
 // router logits, or by a launch of their own without a router.
@@ -503,6 +499,10 @@ static bool direct_routes(const oco_experts *w, uint32_t tokens) {
            plan_desc_words(routes, w->experts, MOE_T) * 4 > align256((uint64_t)tokens * w->hidden * 2);
 }
 
+// The layer after the router logits.  With `logits`, the experts are
+// selected on the device (ids/probs are written): where one route makes a tile
+// inside the routed gate/up kernel (expert_expand's selection), else beside the
+// route plan, or before it by a launch of its own (route_plan_launch).
 static int experts_apply(const oco_experts *w, const void *x, oco_dtype x_dtype, uint32_t *ids, float *probs,
                          const float *logits, uint32_t tokens, uint16_t *out, float *routed, void *workspace,
                          uint64_t workspace_bytes, hipStream_t s, const char *who, bool split_done = false) {

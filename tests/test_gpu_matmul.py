@@ -107,20 +107,22 @@ def test_matmul_prefill_shapes(lib, fmt, n, k):
 @pytest.mark.parametrize("fmt,n,k", [(12, 12288, 4096), (14, 4096, 12288), (8, 4096, 4096)])
 def test_matmul_dense_prefill_bench_shapes(lib, fmt, n, k):
     """The dense prefill bench configurations as the bench runs them (its
-    weight and activation seeds, 512 bf16 tokens, bf16 output, the vendor
-    path): every 32nd row against the fp64 oracle, within 2e-3 and the
+    weight and activation seeds, 512 bf16 tokens, bf16 output), on the kernel
+    the choice takes and on the pass + GEMM: every 32nd row against the fp64 oracle, within 2e-3 and the
     per-element half-operand bound with the output rounding."""
     from oco_amd import synth
     m = 512
     say("matmul dense prefill bench shape", fmt, n, k)
     w = synth.weights(fmt, n, k, 7)
     x = synth.bf16_bits(synth.activations(8, m * k)).reshape(m, k)
-    assert lib.matmul_workspace(fmt, lib.Matrix(k, n, m, 0, 1, 1, 0)) > 0  # the vendor path
-    got = _run_dense(lib, fmt, w, x, m, n, k, y_bf16=True)[::32]
     exact, _ = O.matmul_reference(fmt, w, x[::32], n, k, half_operands=False)
     half, mag = O.matmul_reference(fmt, w, x[::32], n, k, half_operands=True)
-    assert rel_l2(got, exact) <= 2e-3
-    assert np.all(np.abs(got - half) <= O.roundoff_bound(half, mag, k, True))
+    for values, kernel in (((), lib.MatmulKernel.PANEL if fmt == 12 else lib.MatmulKernel.GEMM), ((1,), lib.MatmulKernel.GEMM)):
+        with lib.overridden(lib.Knob.MATMUL_VENDOR, values):
+            assert lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 0), y_dtype=lib.DType.BF16)[0] == kernel
+            got = _run_dense(lib, fmt, w, x, m, n, k, y_bf16=True)[::32]
+        assert rel_l2(got, exact) <= 2e-3
+        assert np.all(np.abs(got - half) <= O.roundoff_bound(half, mag, k, True))
 
 
 def test_matmul_bias_and_bf16_output(lib):
@@ -241,9 +243,8 @@ def test_matmul_mxfp4_tails(lib, m, n, k):
         assert np.array_equal(again.view(np.uint32), first.view(np.uint32))
 
 
-# Formats with f16 operands: at 64 activation rows and more (n % 4 == 0)
-# they take the dequantize pass and the vendor GEMM unless the knob says
-# otherwise.  Both paths run the same operand bits, so both meet the
+# Formats with f16 operands: the fused tiles and the dequantize pass + vendor
+# GEMM, as the knob asks.  Both paths run the same operand bits, so both meet the
 # half-operand roundoff bound per element.
 VENDOR_FORMATS = [P.Q8_0, P.Q4_K, P.Q6_K, P.Q5_K, P.Q4_0, P.Q4_1, 1, 0]
 
@@ -589,10 +590,12 @@ def test_matmul_q4_odd_rows_take_no_gain(lib, fmt, m):
 @pytest.mark.parametrize("m", [31, 32, 33])
 @pytest.mark.parametrize("fmt", [P.Q4_K, P.Q8_0])
 def test_matmul_around_the_vendor_threshold(lib, fmt, m):
-    """Either side of the 32-row switch between the fused tiles and the
-    vendor GEMM: both within the half-operand bound, bias and bf16 output."""
+    """Either side of the 32-row switch between the few-row kernel and the ones
+    with a workspace: within the half-operand bound, bias and bf16 output."""
     from oco_amd import synth
     n, k = 260, 512
+    route = lib.matmul_route(fmt, lib.Matrix(k, n, m, 0, 1, 1, 1), y_dtype=lib.DType.BF16)[0]
+    assert route == (lib.MatmulKernel.FEW_ROWS if m < 32 else lib.MatmulKernel.PANEL)
     w = synth.weights(fmt, n, k, seed=101)
     x = synth.bf16_bits(synth.activations(102, m * k)).reshape(m, k)
     bias = np.random.default_rng(103).normal(size=n).astype(np.float32)
